@@ -46,6 +46,7 @@
 #include "eff_device.h"
 #include "eff_formats.h"
 #include "eff_kernels.h"
+#include "eff_sx.h"
 
 namespace eff {
 
@@ -54,20 +55,6 @@ static __constant__ uint64_t c_grid_sx[256] = {
 };
 
 namespace {
-
-typedef _Float16 half2v __attribute__((ext_vector_type(2)));
-
-
-// Types with group minima (their group sums of x form a 17th slot)
-template <int TYPE>
-constexpr bool sx_mins() {
-  return TYPE == Q2_K || TYPE == Q4_K;
-}
-
-template <int TYPE>
-constexpr uint32_t sx_slots() {  // x slots of 1 KB per (token tile, block): 16 steps (+ group sums)
-  return sx_mins<TYPE>() ? 17u : 16u;
-}
 
 // ---------------------------------------------------------------------------
 // x -> fp16 hi/lo parts. A wave per (token, block); lane l holds x values
@@ -238,35 +225,6 @@ __device__ __forceinline__ void sx_fill8(const float4 (&v)[8], uint32_t lane, ui
 // block's first byte at byte offset `a` of r[0]); `step` returns the 8
 // weights u of step s (k 16 s + 8 h .. + 7 of the block) for lane half h.
 
-// 4 bytes b (each < 1024 after the caller's masking) -> 1024 + b as fp16 pairs
-__device__ __forceinline__ half2v h1024_lo(uint32_t v) {
-  return __builtin_bit_cast(half2v, __builtin_amdgcn_perm(0x64646464u, v, 0x04010400u));
-}
-__device__ __forceinline__ half2v h1024_hi(uint32_t v) {
-  return __builtin_bit_cast(half2v, __builtin_amdgcn_perm(0x64646464u, v, 0x04030402u));
-}
-
-// 8 unsigned bytes q (v0: q0..q3, v1: q4..q7) -> sc * q as fp16, exact
-// (sc * q < 2048; the fused multiply-add rounds once: (1024 + q) sc - 1024 sc)
-__device__ __forceinline__ half8 dec_scaled(uint32_t v0, uint32_t v1, uint32_t sc) {
-  const _Float16 s = (_Float16)(float)sc, o = (_Float16)(-1024.f * (float)sc);
-  const half2v s2 = {s, s}, o2 = {o, o};
-  const half2v a = __builtin_elementwise_fma(h1024_lo(v0), s2, o2);
-  const half2v b = __builtin_elementwise_fma(h1024_hi(v0), s2, o2);
-  const half2v c = __builtin_elementwise_fma(h1024_lo(v1), s2, o2);
-  const half2v d = __builtin_elementwise_fma(h1024_hi(v1), s2, o2);
-  return half8{a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y};
-}
-
-// 8 unsigned bytes -> fp16 (exact below 1024)
-__device__ __forceinline__ half8 dec_plain(uint32_t v0, uint32_t v1) {
-  const half2v o2 = {(_Float16)-1024.f, (_Float16)-1024.f};
-  const half2v a = h1024_lo(v0) + o2, b = h1024_hi(v0) + o2, c = h1024_lo(v1) + o2, d = h1024_hi(v1) + o2;
-  return half8{a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y};
-}
-
-__device__ __forceinline__ uint32_t byte_of(const uint32_t *w, uint32_t i) { return (w[i >> 2] >> (8u * (i & 3u))) & 0xFFu; }
-
 template <int TYPE> struct SxW;
 
 // Q2_K, 84 bytes: scales[16] | qs[64] | d | dmin (kernels.wgsl.js:194-222).
@@ -418,15 +376,6 @@ template <> struct SxW<IQ2_XXS> {
     return half8{v0.x, v0.y, v1.x, v1.y, v2.x, v2.y, v3.x, v3.y};
   }
 };
-
-// 8 signed bytes q -> q as fp16 (exact): 1024 + (q + 128) - 1152
-__device__ __forceinline__ half8 dec_signed(uint32_t v0, uint32_t v1) {
-  const half2v o2 = {(_Float16)-1152.f, (_Float16)-1152.f};
-  v0 ^= 0x80808080u;
-  v1 ^= 0x80808080u;
-  const half2v a = h1024_lo(v0) + o2, b = h1024_hi(v0) + o2, c = h1024_lo(v1) + o2, d = h1024_hi(v1) + o2;
-  return half8{a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y};
-}
 
 // Q8_0, 256 weights = 8 blocks of 34 bytes, d | q[32] (kernels.wgsl.js:154-160).
 // Step s: block s / 2, quants 16 (s % 2) + 8 h .. + 7 (bytes 34 (s / 2) + 2 +
@@ -864,8 +813,10 @@ __global__ __launch_bounds__(NW * 64) void k_sx(WeightView wv, const uint8_t *__
 // Token tiles of 16 per wave (tt) and token groups (grid y); the x scratch
 // covers groups * tt tiles (tokens past `tokens` are zero).
 struct SxPlan {
-  // cfg 0: 32 rows x 8 waves; 1: 64 rows x 4 waves; ksl: k slices per row tile
+  // cfg 0: 32 rows x 8 waves; 1: 64 rows x 4 waves; ksl: k slices per row tile;
+  // shared: the LDS-shared tiles (k_sxt) instead, in ksl slices
   uint32_t tt, cfg, groups, row_tiles, nbw, ksl;
+  bool shared;
 };
 
 // The types folded per group of steps (Q8_0, Q8_0R, Q6_K) take at most 2
@@ -876,6 +827,58 @@ void sx_tiles(int type, uint32_t tokens, uint32_t &tt, uint32_t &groups) {
   const uint32_t ttn = (tokens + 15u) / 16u;
   tt = ttn <= 1u ? 1u : ttn <= 2u || sx_tt_max(type) == 2u ? 2u : 4u;
   groups = (ttn + tt - 1u) / tt;
+}
+
+// Token tiles of the x scratch: whole groups of every plan of the type (4
+// tiles for the LDS-shared tiles, which no plan takes below 33 tokens).
+uint32_t sx_tile_count(int type, uint32_t tokens) {
+  uint32_t tt, groups;
+  sx_tiles(type, tokens, tt, groups);
+  return tokens > 32u ? (tt * groups + 3u) / 4u * 4u : tt * groups;
+}
+
+// k slices of the LDS-shared tiles (k_sxt) where they are estimated to be
+// faster than the plan of k_sx, else 0. Both times (us) are linear in a CU's
+// rounds of workgroups and in the blocks of k a round walks, plus the slices'
+// sums; the coefficients are least-squares fits (5% and 7% rms error) to
+// timings of both kernels at 90 shapes a type from 1024 to 14336 rows, k = 1024
+// to 8192 and 40 to 2048 tokens (k_sxt in 1 to 8 slices). The choice is 0.2%
+// above the faster of the two summed over them, and 16% (Q4_K), 43% (Q6_K), 12%
+// (IQ2_XXS) and 20% (Q2_K) below k_sx alone. us, k_sx / k_sxt: Q4_K 8192 x 2048
+// at 512 tokens 71.7 / 54.4, 4096 x 2048 at 1000 71.9 / 55.3, 8192 x 8192 at 512
+// 224 / 161, but 6144 x 1024 at 256 21.3 / 23.7 and 8192 x 4096 at 96 32.8 /
+// 38.1 (4 slices); Q6_K 8192 x 2048 at 512 130 / 65, 2048 x 8192 at 300 83 / 52
+// (3 slices), 2048 x 2048 at 128 13.0 / 17.0.
+uint32_t sxt_choose(const WeightView &wv, uint32_t tokens, double rounds, uint32_t walk, bool sliced) {
+  struct Fit {
+    int type;
+    double sx[5];    // launch, per round, per round and block of a token tile, if sliced, per 1e6 values of x
+    double sxt[6];   // launch, per round, per round and pair of blocks, if sliced, per 1e6 sums of all slices, x
+  };
+  static const Fit fits[] = {{Q4_K, {4.08, 1.90, 0.210, 2.23, 3.54}, {1.12, 9.20, 6.94, 4.03, 1.79, 2.72}},
+                             {Q6_K, {4.21, 2.58, 0.350, 2.62, 3.25}, {2.04, 6.12, 5.00, 1.59, 1.85, 3.28}},
+                             {Q2_K, {4.04, 1.71, 0.210, 2.13, 3.36}, {2.16, 7.63, 6.21, 2.82, 1.82, 2.93}},
+                             {IQ2_XXS, {4.64, 1.53, 0.205, 2.29, 3.11}, {2.39, 5.55, 4.15, 1.65, 1.52, 3.12}}};
+  if (tokens <= 32u) return 0u;   // the x scratch then holds less than the kernel's 64 tokens
+  const uint64_t nb = wv.k / 256u, xb = (uint64_t)sx_tile_count(wv.type, tokens) * nb * 17u * 1024u;
+  if (xb >= (1ull << 32) || (uint64_t)wv.rows * (wv.k / 256u) * 210u >= (1ull << 32)) return 0u;   // 32-bit offsets
+  for (const Fit &f : fits) {
+    if (f.type != wv.type) continue;
+    const double xk = 1e-6 * tokens * wv.k, out = 1e-6 * tokens * wv.rows;
+    double best = 0.95 * (f.sx[0] + rounds * (f.sx[1] + f.sx[2] * walk) + (sliced ? f.sx[3] : 0.0) + f.sx[4] * xk);
+    const uint32_t rt = sxt_row_tile(wv.type);
+    const uint64_t tiles = (uint64_t)((wv.rows + rt - 1u) / rt) * ((tokens + 63u) / 64u);
+    uint32_t ksl = 0u;
+    for (uint32_t s : {1u, 2u, 3u, 4u, 6u, 8u}) {
+      if (s > 1u && (tiles * s > 640u || nb / s < 2u)) break;
+      const uint64_t r = (tiles * s + 255u) / 256u, pairs = ((nb + s - 1u) / s + 1u) / 2u;
+      const double t = f.sxt[0] + (double)r * (f.sxt[1] + f.sxt[2] * (double)pairs) +
+                       (s > 1u ? f.sxt[3] + f.sxt[4] * out * s : 0.0) + f.sxt[5] * xk;
+      if (t < best) best = t, ksl = s;
+    }
+    return ksl;
+  }
+  return 0u;
 }
 
 SxPlan sx_plan(const WeightView &wv, uint32_t tokens, int cfg, uint32_t ksl_opt) {
@@ -921,6 +924,11 @@ SxPlan sx_plan(const WeightView &wv, uint32_t tokens, int cfg, uint32_t ksl_opt)
   p.ksl = ksl_opt ? ksl_opt : cfg == 3 ? 2u : ks_auto;
   p.ksl = max(1u, min(p.ksl, nb));
   p.nbw = ((nb + p.ksl - 1u) / p.ksl + nw - 1u) / nw;
+  // the LDS-shared tiles, where they are estimated to be the faster
+  const double rounds = p.ksl > 1u ? (p.cfg ? 1.75 : 1.0) * ((wgs * p.ksl + 255u) / 256u) : p.cfg ? t64 : t32;
+  const uint32_t shared = cfg == 0 ? sxt_choose(wv, tokens, rounds, (nb + p.ksl - 1u) / p.ksl * p.tt, p.ksl > 1u) : 0u;
+  p.shared = shared != 0u;
+  if (p.shared) p.ksl = max(1u, min(ksl_opt ? ksl_opt : shared, nb));
   return p;
 }
 
@@ -976,6 +984,7 @@ template <int TYPE>
 hipError_t sx_main(const WeightView &wv, const uint8_t *xa, uint32_t tiles, float *y, uint32_t tokens,
                    const SxPlan &p, void *sk, hipStream_t s) {
   const float *xp = (const float *)(xa + (uint64_t)tiles * (wv.k / 256u) * sx_slots<TYPE>() * 1024u);
+  if (p.shared) return launch_sxt(wv, xa, xp, tiles, y, tokens, p.ksl, sk, s);
   switch (p.tt) {
     case 1: return sx_cfg<TYPE, 1>(wv, xa, xp, y, tokens, p, sk, s);
     case 2: return sx_cfg<TYPE, 2>(wv, xa, xp, y, tokens, p, sk, s);
@@ -991,7 +1000,7 @@ hipError_t sx_type(const WeightView &wv, const float *x, float *y, uint32_t toke
   const SxPlan p = sx_plan(wv, tokens, cfg, ksl_opt);
   if constexpr (TYPE == Q2_K || TYPE == IQ2_XXS)
     if (sx_fx(TYPE, tokens, cfg, p, wv.k)) return sx_go_fx<TYPE>(wv, x, y, tokens, p, s);
-  const uint32_t tiles = p.groups * p.tt, nb = wv.k / 256u;   // blocks of 256 weights
+  const uint32_t tiles = sx_tile_count(TYPE, tokens), nb = wv.k / 256u;   // blocks of 256 weights
   uint8_t *xa = scratch;
   float *xp = (float *)(scratch + (uint64_t)tiles * nb * sx_slots<TYPE>() * 1024u);
   hipLaunchKernelGGL((k_sx_prep<TYPE>), dim3(nb, tiles * 4u), dim3(256), 0, s, x, tokens, wv.k, xa, xp);
@@ -1013,15 +1022,14 @@ bool sx_applies(const WeightView &wv, uint32_t tokens) {
 }
 
 size_t sx_x_bytes(int type, uint32_t tokens, uint32_t k) {
-  uint32_t tt, groups;
-  sx_tiles(type, tokens, tt, groups);
-  const uint64_t tiles = (uint64_t)tt * groups, nb = k / 256u;
+  const uint64_t tiles = sx_tile_count(type, tokens), nb = k / 256u;
   const uint32_t slots = type == Q2_K || type == Q4_K ? 17u : 16u;   // sx_slots
   return (size_t)(tiles * nb * slots * 1024u + tiles * nb * 64u);
 }
 
 size_t sx_sk_bytes(const WeightView &wv, uint32_t tokens, int cfg, uint32_t ksl_opt) {
   const SxPlan p = sx_plan(wv, tokens, cfg, ksl_opt);
+  if (p.shared) return sxt_sk_bytes(wv, tokens, p.ksl);
   if (p.ksl < 2u || sx_fx(wv.type, tokens, cfg, p, wv.k)) return 0;
   const uint64_t ne = (uint64_t)p.tt * (p.cfg ? 2u : 1u) * 512u;   // sums per workgroup
   return kSliceCntBytes + (size_t)((uint64_t)p.row_tiles * p.groups * p.ksl * ne * 4u);

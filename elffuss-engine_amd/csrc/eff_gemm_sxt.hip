@@ -1,0 +1,689 @@
+// Split-x product over LDS-shared tiles, for prompts of the K and IQ types:
+// the arithmetic of eff_gemm_sx.hip (x as fp16 hi and lo parts, integer weights
+// exact in fp16, f32 sums, one scale per block of 256), from the same prepared
+// x, for token counts where reading x bounds that kernel.
+//
+// What bounds k_sx at many tokens: every wave reads its x fragments from L2 by
+// itself, 0.5 KB per matrix instruction with 64 rows per wave: 64 bytes per
+// clock and CU with the matrix cores busy, all that a CU's vector memory path
+// delivers. Here a workgroup's waves share x through LDS.
+//
+// Workgroup: 8 waves (2 per SIMD) over 64 tokens x 256 rows, as 4 groups of 64
+// rows x 2 slices of k (slice z takes every second block of 256). A wave holds
+// 2 x 2 tiles of 32 tokens x 32 rows: per step of 16 k it reads 2 lo and 2 hi
+// fragments of x (4 KB) for 8 v_mfma_f32_32x32x16_f16, decodes its 2 weight
+// fragments in registers, and adds lo and hi into one accumulator per tile,
+//   D += u lo, D += u hi,
+// folded once per block: acc += D d p (p: x's block scales). x flows in groups of 4 steps through two
+// LDS buffers (direct-to-LDS loads a group ahead, one barrier per group); the
+// raw weights of the next block are loaded into a region of LDS of the wave's
+// own while the present block's are in registers.
+//
+// Errors against 64 bits are those of k_sx or smaller (2048 x 8192 to 8192 x
+// 2048, 300-512 tokens): a D that takes lo and hi parts is rounded twice as
+// often as one of the hi parts alone (1.25 times the error). Q4_K and Q2_K make
+// up for it with smaller sums: u = sc (q - 8) and sc (q - 1.5) instead of sc q,
+// and D opens with the group sums' terms, -(dmin / d) sum mn_g S_g + 8 (1.5)
+// sum sc_g S_g (1.9e-7 against 3.2e-7, 1.8e-7 against 2.1e-7). IQ2_XXS and Q6_K
+// keep the lo parts in accumulators of their own, which leaves registers for
+// one row tile per wave (1.3e-7 as before; Q6_K 1.2e-7 against 1.7e-7, its hi
+// parts in two sums of 8 steps).
+//
+// Q6_K: u = sc (q - 32) has up to 13 bits, so its fp16 rounding v = fp16(u) is
+// off by r = u - v in {-1, 0, 1}, and only where |u| > 2048. The product takes
+// hi and lo times v plus hi times r; what is left out, lo times r, is below
+// 2^-22 of the term. Three matrix instructions instead of two, and one fold per
+// block instead of 16 (whose 24 vector instructions per matrix instruction
+// bound k_sx there).
+//
+// What bounds it now: with random operands the matrix cores hold 1.4 PFLOP/s
+// beside 6 vector instructions per instruction (the clock falls from 2.4 to 1.5
+// GHz); a round of workgroups walks 512 k of 64 x 256 outputs per CU in 7 us
+// (Q4_K, 1.28 PFLOP/s of hi and lo products) after about 4 us for its first
+// loads, and ends with all of its y written at once, another 4. us, k_sx before
+// and this kernel, both with the preparation of x: Q4_K 8192 x 2048 at 512
+// tokens 63.8 / 48.8, Q6_K 2048 x 8192 at 300 78.0 / 50.0, Q4_K 4096 x 4096 at
+// 1000 125 / 91.
+#include <hip/hip_runtime.h>
+#include <math.h>
+#include <stdint.h>
+
+#include "../../include/elffuss_amd.h"
+#include "eff_device.h"
+#include "eff_formats.h"
+#include "eff_kernels.h"
+#include "eff_sx.h"
+
+namespace eff {
+
+static __constant__ uint64_t c_grid_sxt[256] = {
+#include "iq2xxs_grid.inc"
+};
+
+namespace {
+
+// The raw weights of 32 rows, unit by unit (a block of 256 weights, or half of
+// one): NI direct-to-LDS loads of 1 KB, whose lane (row j, half h) brings 16
+// bytes; 16-byte piece P of row j is then at 512 P + 16 j of the region. `fetch`
+// issues the loads of unit `un` of the block at byte `bo` of the lane's row,
+// `take` reads the unit's weights into registers, `step` decodes the 8 weights
+// of the lane in step s of the unit (k 16 s + 8 h .. + 7) to exact fp16.
+template <int TYPE> struct SxtW;
+
+__device__ __forceinline__ uint64_t lds64(const uint8_t *p) { return *(const uint64_t *)p; }
+__device__ __forceinline__ uint32_t lds32(const uint8_t *p) { return *(const uint32_t *)p; }
+
+// 8 bytes b (v0, v1) -> (1024 + b) (sc f) + sc o as fp16: every operand and the
+// result are exact, so the fused multiply-add is.
+__device__ __forceinline__ half8 dec_centred(uint32_t v0, uint32_t v1, uint32_t sc, float f, float o) {
+  const _Float16 s = (_Float16)((float)sc * f), c = (_Float16)((float)sc * o);
+  const half2v s2 = {s, s}, c2 = {c, c};
+  const half2v a = __builtin_elementwise_fma(h1024_lo(v0), s2, c2);
+  const half2v b = __builtin_elementwise_fma(h1024_hi(v0), s2, c2);
+  const half2v e = __builtin_elementwise_fma(h1024_lo(v1), s2, c2);
+  const half2v g = __builtin_elementwise_fma(h1024_hi(v1), s2, c2);
+  return half8{a.x, a.y, b.x, b.y, e.x, e.y, g.x, g.y};
+}
+
+// The block's scale d and the ratio its minima's sums are scaled by. A block
+// with d = 0 keeps its minima: its u are zeroed (by the caller) and the scale is
+// dmin itself.
+__device__ __forceinline__ void min_ratio(float &d, float dm, float &ratio) {
+  ratio = d != 0.f ? -dm / d : -1.f;
+  d = d != 0.f ? d : dm;
+}
+
+// Q4_K, 144 bytes: d | dmin | scales[12] | qs[128]. Piece 0: the header; pieces
+// 1 + 2 c + m: qs of 64-weight chunk c, bytes 16 m .. (piece 9 is the next
+// block's and not read).
+template <> struct SxtW<Q4_K> {
+  static constexpr uint32_t NI = 5, UNITS = 1, BB = 144;
+  static constexpr bool REM = false;
+  static constexpr int FB = 2;          // tiles of 32 rows per wave
+  static constexpr bool SEP = false;
+  uint32_t q[16], sc[2], mi[2];
+  float d, ratio;
+  __device__ static void fetch(rsrc_t src, const uint8_t *reg, uint32_t voff, uint32_t bo, int, uint32_t h) {
+#pragma unroll
+    for (uint32_t i = 0; i < NI; ++i) dma16(src, reg + 1024u * i, voff + 16u * h, bo + 32u * i);
+  }
+  __device__ void take(const uint8_t *reg, int, uint32_t j, uint32_t h, uint32_t) {
+    const u32x4 hd = *(const u32x4 *)(reg + 16u * j);
+#pragma unroll
+    for (int p = 0; p < 8; ++p) {
+      const uint64_t v = lds64(reg + 512u * (p + 1) + 16u * j + 8u * h);
+      q[2 * p] = (uint32_t)v;
+      q[2 * p + 1] = (uint32_t)(v >> 32);
+    }
+    d = h2f(hd.x & 0xFFFFu);
+    const uint32_t keep = d != 0.f ? 0x3F3F3F3Fu : 0u;
+    sc[0] = hd.y & keep;
+    mi[0] = hd.z & 0x3F3F3F3Fu;
+    sc[1] = ((hd.w & 0x0F0F0F0Fu) | ((hd.y >> 2) & 0x30303030u)) & keep;
+    mi[1] = ((hd.w >> 4) & 0x0F0F0F0Fu) | ((hd.z >> 2) & 0x30303030u);
+    min_ratio(d, 32.f * h2f(hd.x >> 16), ratio);  // group sums are stored divided by 32
+  }
+  // u = sc (q - 8), from the nibble in a byte's high half: (1024 + 16 q) sc / 16 - 72 sc
+  __device__ half8 step(int s, uint32_t, const uint8_t *) const {
+    const int c = s >> 2, nib = (s >> 1) & 1, m = s & 1;
+    const uint32_t w0 = q[4 * c + 2 * m], w1 = q[4 * c + 2 * m + 1];
+    return dec_centred((nib ? w0 : w0 << 4) & 0xF0F0F0F0u, (nib ? w1 : w1 << 4) & 0xF0F0F0F0u,
+                       byte_of(sc, (uint32_t)s >> 1), 0.0625f, -72.f);
+  }
+  // 8 minima and 8 scales: one instruction takes the sums' hi parts in k 0..7, lo in 8..15
+  static constexpr uint32_t MSTEP = 1;
+  __device__ half8 mins(uint32_t) const { return dec_plain(mi[0], mi[1]); }
+  __device__ half8 centre(uint32_t) const { return dec_plain(sc[0], sc[1]) * (_Float16)256.f; }   // 8 x 32 sc
+};
+
+// Q2_K, 84 bytes: scales[16] | qs[64] | d | dmin. Pieces 0: scales, 1 + 2 n + m:
+// qs of the half n, bytes 16 m .., 5: d and dmin.
+template <> struct SxtW<Q2_K> {
+  static constexpr uint32_t NI = 3, UNITS = 1, BB = 84;
+  static constexpr bool REM = false;
+  static constexpr int FB = 2;          // tiles of 32 rows per wave
+  static constexpr bool SEP = false;
+  uint32_t q[8], sc[4];
+  float d, ratio;
+  __device__ static void fetch(rsrc_t src, const uint8_t *reg, uint32_t voff, uint32_t bo, int, uint32_t h) {
+#pragma unroll
+    for (uint32_t i = 0; i < NI; ++i) dma16(src, reg + 1024u * i, voff + 16u * h, bo + 32u * i);
+  }
+  __device__ void take(const uint8_t *reg, int, uint32_t j, uint32_t h, uint32_t) {
+    const u32x4 s = *(const u32x4 *)(reg + 16u * j);
+    const uint32_t w = lds32(reg + 512u * 5u + 16u * j);
+    d = h2f(w & 0xFFFFu);
+    const uint32_t kp = d != 0.f ? 0xFFFFFFFFu : 0xF0F0F0F0u;
+    sc[0] = s.x & kp; sc[1] = s.y & kp; sc[2] = s.z & kp; sc[3] = s.w & kp;
+#pragma unroll
+    for (int p = 0; p < 4; ++p) {
+      const uint64_t v = lds64(reg + 512u * (p + 1) + 16u * j + 8u * h);
+      q[2 * p] = (uint32_t)v;
+      q[2 * p + 1] = (uint32_t)(v >> 32);
+    }
+    min_ratio(d, 16.f * h2f(w >> 16), ratio);  // group sums are stored divided by 16
+  }
+  // u = sc (q - 1.5), from the 2 bits at a byte's top: (1024 + 64 q) sc / 64 - 17.5 sc
+  __device__ half8 step(int s, uint32_t, const uint8_t *) const {
+    const int n = s >> 3, g = (s >> 1) & 3, m = s & 1;
+    return dec_centred((q[4 * n + 2 * m] << (6 - 2 * g)) & 0xC0C0C0C0u,
+                       (q[4 * n + 2 * m + 1] << (6 - 2 * g)) & 0xC0C0C0C0u, byte_of(sc, (uint32_t)s) & 15u, 0.015625f,
+                       -17.5f);
+  }
+  static constexpr uint32_t MSTEP = 2;   // 16 minima: lo, then hi
+  __device__ half8 mins(uint32_t h) const {
+    const uint32_t w0 = h ? sc[2] : sc[0], w1 = h ? sc[3] : sc[1];
+    return dec_plain((w0 >> 4) & 0x0F0F0F0Fu, (w1 >> 4) & 0x0F0F0F0Fu);
+  }
+  __device__ half8 centre(uint32_t h) const {   // 1.5 x 16 sc
+    return dec_plain((h ? sc[2] : sc[0]) & 0x0F0F0F0Fu, (h ? sc[3] : sc[1]) & 0x0F0F0F0Fu) * (_Float16)24.f;
+  }
+};
+
+// IQ2_XXS, 66 bytes: d | 8 x (4 grid indices, 4 sign fields and a scale), from
+// the 4-byte floor of the block's first byte (`a`: 0 or 2 bytes before it). A
+// lane keeps, per step, its grid index and sign field, and the scales. The grid
+// (256 x 8 bytes) is in LDS; the sign bits come from the field and its parity
+// by shifts.
+template <> struct SxtW<IQ2_XXS> {
+  static constexpr uint32_t NI = 3, UNITS = 1, BB = 66;
+  static constexpr bool REM = false;
+  static constexpr int FB = 1;          // tiles of 32 rows per wave
+  static constexpr bool SEP = true;
+  uint32_t g[8], sc;   // g[i]: steps 2 i and 2 i + 1, 16 bits each: index | field << 8
+  float d, ratio;
+  __device__ static void fetch(rsrc_t src, const uint8_t *reg, uint32_t voff, uint32_t bo, int, uint32_t h) {
+    const uint32_t v = ((voff + bo) & ~3u) + 16u * h;
+#pragma unroll
+    for (uint32_t i = 0; i < NI; ++i) dma16(src, reg + 1024u * i, v, 32u * i);
+  }
+  __device__ void take(const uint8_t *reg, int, uint32_t j, uint32_t h, uint32_t a) {
+    uint32_t w[20];
+#pragma unroll
+    for (int p = 0; p < 5; ++p) {
+      const u32x4 v = *(const u32x4 *)(reg + 512u * p + 16u * j);
+      w[4 * p] = v.x; w[4 * p + 1] = v.y; w[4 * p + 2] = v.z; w[4 * p + 3] = v.w;
+    }
+    const uint32_t sel = a ? 0x07060504u : 0x05040302u;
+    sc = 0u;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      const uint32_t a0 = __builtin_amdgcn_perm(w[2 * i + 1], w[2 * i], sel) >> (8u * h);
+      const uint32_t a1 = __builtin_amdgcn_perm(w[2 * i + 2], w[2 * i + 1], sel);
+      sc |= (a1 >> 28) << (4 * i);
+      g[i] = (a0 & 0x00FF00FFu) | (__builtin_amdgcn_ubfe(a1, 7u * h, 7u) << 8) |
+             (__builtin_amdgcn_ubfe(a1, 14u + 7u * h, 7u) << 24);
+    }
+    d = 0.125f * h2f(a ? (w[0] >> 16) : (w[0] & 0xFFFFu));
+    ratio = 0.f;
+  }
+  __device__ half8 step(int s, uint32_t, const uint8_t *tab) const {
+    const int b = 16 * (s & 1);
+    const uint64_t e = *(const uint64_t *)(tab + 8u * __builtin_amdgcn_ubfe(g[s >> 1], b, 8));
+    const uint32_t f = __builtin_amdgcn_ubfe(g[s >> 1], b + 8, 7);
+    const uint32_t sg = f | ((uint32_t)__builtin_popcount(f) << 7);   // bits 0..7; the eighth makes the parity even
+    const half8 v = dec_scaled((uint32_t)e, (uint32_t)(e >> 32), 2u * __builtin_amdgcn_ubfe(sc, 4 * (s >> 1), 4) + 1u);
+    u32x4 o = __builtin_bit_cast(u32x4, v);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      // sign bits 2 i and 2 i + 1 to bits 15 and 31 (the values are not negative)
+      const uint32_t m = (sg << (15 - 2 * i)) | (sg << (30 - 2 * i));
+      o[i] |= m & 0x80008000u;
+    }
+    return __builtin_bit_cast(half8, o);
+  }
+  __device__ half8 mins(uint32_t) const { return half8{0, 0, 0, 0, 0, 0, 0, 0}; }
+};
+
+// Q6_K, 210 bytes: ql[128] | qh[64] | scales[16] (int8) | d, half a block (128
+// weights) per unit n, from the 4-byte floor of the block's first byte. Pieces
+// 0..4: ql bytes 64 n .. + 79, 5..7: qh bytes 128 + 32 n .. + 47, 8..9: scales
+// and d (bytes 192 .. 223; each run one piece longer than its bytes where the
+// floor moves it by 2).
+template <> struct SxtW<Q6_K> {
+  static constexpr uint32_t NI = 5, UNITS = 2, BB = 210;
+  static constexpr bool REM = true;
+  static constexpr int FB = 1;          // tiles of 32 rows per wave
+  static constexpr bool SEP = true;
+  uint32_t ql[8], qh[4], sc[2];
+  float d, ratio;
+  __device__ static void fetch(rsrc_t src, const uint8_t *reg, uint32_t voff, uint32_t bo, int un, uint32_t h) {
+    const uint32_t v = (voff + bo) & ~3u, n = (uint32_t)un, vh = v + 16u * h;
+    dma16(src, reg, vh, 64u * n);
+    dma16(src, reg + 1024u, vh, 64u * n + 32u);
+    dma16(src, reg + 2048u, v + (h ? 128u + 32u * n : 64u + 64u * n), 0u);
+    dma16(src, reg + 3072u, vh, 144u + 32u * n);
+    dma16(src, reg + 4096u, vh, 192u);
+  }
+  __device__ void take(const uint8_t *reg, int un, uint32_t j, uint32_t h, uint32_t a) {
+    const uint8_t *p0 = reg + 16u * j + 8u * h;             // the lane's 8 bytes of a piece
+    const uint8_t *p1 = reg + 16u * j + (h ? 512u : 8u);    // and the dword after them
+    auto get = [&](int p, uint32_t &o0, uint32_t &o1) {
+      const uint64_t w = lds64(p0 + 512 * p);
+      const uint32_t w2 = lds32(p1 + 512 * p);
+      o0 = __builtin_amdgcn_alignbyte((uint32_t)(w >> 32), (uint32_t)w, a);
+      o1 = __builtin_amdgcn_alignbyte(w2, (uint32_t)(w >> 32), a);
+    };
+#pragma unroll
+    for (int p = 0; p < 4; ++p) get(p, ql[2 * p], ql[2 * p + 1]);
+#pragma unroll
+    for (int p = 0; p < 2; ++p) get(5 + p, qh[2 * p], qh[2 * p + 1]);
+    const uint8_t *ps = reg + 512u * 8u + 16u * j;
+    const uint64_t s01 = lds64(ps + 8 * un);
+    const uint32_t s2 = lds32(un ? ps + 512 : ps + 8), w = lds32(ps + 512);
+    sc[0] = __builtin_amdgcn_alignbyte((uint32_t)(s01 >> 32), (uint32_t)s01, a);
+    sc[1] = __builtin_amdgcn_alignbyte(s2, (uint32_t)(s01 >> 32), a);
+    d = h2f(a ? (w >> 16) : (w & 0xFFFFu));
+    ratio = 0.f;
+  }
+  // step s of the unit (0..7): v = fp16(sc (q - 32)) and what it is off by
+  __device__ half8 step2(int s, half8 &rem) const {
+    const int g = s >> 1, m = s & 1, p = 2 * (g & 1) + m, ls = 4 * (g >> 1), hs = 2 * g;
+    const uint32_t u0 = ((ql[2 * p] >> ls) & 0x0F0F0F0Fu) | (((qh[2 * m] >> hs) & 0x03030303u) << 4);
+    const uint32_t u1 = ((ql[2 * p + 1] >> ls) & 0x0F0F0F0Fu) | (((qh[2 * m + 1] >> hs) & 0x03030303u) << 4);
+    const half2v o2 = {(_Float16)-1056.f, (_Float16)-1056.f};   // 1024 + q - 1056 = q - 32
+    const _Float16 c = (_Float16)(float)(int8_t)byte_of(sc, (uint32_t)s);
+    const half2v c2 = {c, c};
+    const half2v e[4] = {h1024_lo(u0) + o2, h1024_hi(u0) + o2, h1024_lo(u1) + o2, h1024_hi(u1) + o2};
+    half8 v;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const half2v t = e[i] * c2, r = __builtin_elementwise_fma(e[i], c2, -t);
+      v[2 * i] = t.x; v[2 * i + 1] = t.y;
+      rem[2 * i] = r.x; rem[2 * i + 1] = r.y;
+    }
+    return v;
+  }
+  __device__ half8 mins(uint32_t) const { return half8{0, 0, 0, 0, 0, 0, 0, 0}; }
+};
+
+// s_waitcnt vmcnt(N) lgkmcnt(0): the loads past the N youngest are in, and
+// every LDS read of this wave has returned.
+template <uint32_t N>
+__device__ __forceinline__ void wait_vm_lds() {
+  static_assert(N < 64, "vmcnt");
+  __builtin_amdgcn_s_waitcnt((int)((N & 15u) | ((N >> 4) << 14) | 0x0070u));
+}
+
+constexpr uint32_t kTokTile = 64;    // tokens per workgroup: 4 tiles of 16 of the prepared x
+
+template <int TYPE>
+constexpr uint32_t sxt_rows() {      // rows per workgroup: 4 groups of 32 FB
+  static_assert(sxt_row_tile(TYPE) == 128u * SxtW<TYPE>::FB, "row tile");
+  return sxt_row_tile(TYPE);
+}
+
+template <int TYPE>
+struct SxtLds {
+  static constexpr uint32_t XG = 2u * 4u * 4096u;                   // 4 steps of 64 tokens, for each k slice
+  static constexpr uint32_t WR = SxtW<TYPE>::NI * 1024u;            // raw weights of 32 rows
+  static constexpr uint32_t TAB = TYPE == IQ2_XXS ? 2048u : 0u;
+  static constexpr uint32_t X0 = TAB, W0 = X0 + 2u * XG, M0 = W0 + 8u * SxtW<TYPE>::FB * WR;
+  static constexpr uint32_t P0 = M0 + (sx_mins<TYPE>() ? 8192u : 0u);   // group sums of a block, for each k slice
+  static constexpr uint32_t LOOP = P0 + 1024u;                      // block scales: 2 blocks x 2 slices x 64 tokens
+  static constexpr uint32_t RED = 8u * 8192u + 16u;                 // the waves' sums handed over
+  static constexpr uint32_t BYTES = LOOP > RED ? LOOP : RED;
+  static_assert(BYTES <= 160u * 1024u, "LDS");
+};
+
+__device__ __forceinline__ float16v mma(half8 a, half8 b, float16v c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
+}
+
+template <int TYPE>
+__global__ __launch_bounds__(512) void k_sxt(WeightView wv, const uint8_t *__restrict__ xa,
+                                             const float *__restrict__ xp, float *__restrict__ y, uint32_t tokens,
+                                             uint32_t xa_bytes, uint32_t xp_bytes, uint32_t row_tiles,
+                                             uint32_t tok_tiles, uint32_t ksl, float *__restrict__ part,
+                                             uint32_t *__restrict__ cnt) {
+  using W = SxtW<TYPE>;
+  using L = SxtLds<TYPE>;
+  constexpr bool MINS = sx_mins<TYPE>();
+  constexpr uint32_t NS = sx_slots<TYPE>();
+  constexpr int FB = W::FB;
+  constexpr uint32_t SU = 16u / W::UNITS;        // steps of a unit
+  constexpr uint32_t WI = FB * W::NI;            // a wave's loads of a unit's weights
+  constexpr uint32_t XI = 4u;                    // and of a group's x
+  __shared__ __align__(16) uint8_t lds[L::BYTES];
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, j = lane & 31u, h = lane >> 5;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), rg = wave & 3u, ks = wave >> 2;
+
+  // Workgroups of one XCD (blockIdx % 8) take a contiguous run of (k slice,
+  // tile) pairs, token tiles fastest: they share weights through its L2.
+  const uint32_t ntiles = row_tiles * tok_tiles, nwg = ntiles * ksl;
+  uint32_t u = blockIdx.x;
+  if (nwg % 8u == 0u) u = (blockIdx.x % 8u) * (nwg / 8u) + blockIdx.x / 8u;
+  const uint32_t z = u / ntiles, lin = u - z * ntiles;
+  const uint32_t tt0 = lin % tok_tiles, r0 = (lin / tok_tiles) * sxt_rows<TYPE>() + 32u * FB * rg;
+  const uint32_t rows = wv.rows, nb = wv.k / 256u;
+  const uint32_t bl = z * nb / ksl, bh = (z + 1u) * nb / ksl, iters = (bh - bl + 1u) / 2u;
+
+  if constexpr (TYPE == IQ2_XXS) {
+    if (tid < 256u) *(uint64_t *)(lds + 8u * tid) = c_grid_sxt[tid];
+  }
+
+  const rsrc_t wsrc = make_rsrc(wv.w, wv.w_bytes), xsrc = make_rsrc(xa, xa_bytes), psrc = make_rsrc(xp, xp_bytes);
+  const uint32_t rb = (uint32_t)wv.row_bytes;
+  uint32_t wrow[FB];
+#pragma unroll
+  for (int f = 0; f < FB; ++f) wrow[f] = min(r0 + 32u * f + j, rows - 1u) * rb;
+  uint8_t *const wreg = lds + L::W0 + wave * FB * L::WR;
+  const uint32_t pvoff = ((4u * tt0 + (lane >> 4)) * nb * 16u + (lane & 15u)) * 4u;
+  const uint32_t xtile = (4u * tt0 + (wave & 3u)) * nb;
+
+  // the block of slice sl in iteration it (loads past the end repeat the last block)
+  auto blk = [&](uint32_t it, uint32_t sl) { return min(bl + 2u * it + sl, bh - 1u); };
+  auto fetch_w = [&](uint32_t it, int un) {
+    const uint32_t b = blk(it, ks);
+#pragma unroll
+    for (int f = 0; f < FB; ++f) W::fetch(wsrc, wreg + f * L::WR, wrow[f], b * W::BB, un, h);
+  };
+  // x of group g (4 steps) of iteration it: 1 KB chunk c = wave + 8 i is
+  // 16-token tile c % 4 of step c / 4 % 4 of slice c / 16
+  auto fetch_x = [&](uint32_t it, uint32_t g) {
+#pragma unroll
+    for (uint32_t i = 0; i < XI; ++i) {
+      const uint32_t s = ((wave >> 2) + 2u * i) & 3u;
+      dma16(xsrc, lds + L::X0 + (g & 1u) * L::XG + (wave + 8u * i) * 1024u, 16u * lane,
+            ((xtile + blk(it, i >> 1)) * NS + 4u * g + s) * 1024u);
+    }
+  };
+  // the group sums (one 1 KB chunk per wave) and block scales of iteration it
+  auto fetch_m = [&](uint32_t it) {
+    if constexpr (MINS)
+      dma16(xsrc, lds + L::M0 + wave * 1024u, 16u * lane, ((xtile + blk(it, wave >> 2)) * NS + 16u) * 1024u);
+    dma4(psrc, lds + L::P0 + (it & 1u) * 512u + ks * 256u, pvoff, blk(it, ks) * 64u);
+  };
+  // the lane's fragment rows: token j of a tile of 32 = row j % 16 of 16-token tile j / 16
+  const uint8_t *const xl = lds + L::X0 + ks * 16384u + (j >> 4) * 1024u + 16u * (32u * h + (j & 15u));
+
+  // [token tile][row tile]; D2: the sums of the lo parts (and of hi times r)
+  // where they are kept apart
+  float16v acc[2][FB], D[2][FB], D2[2][W::SEP ? FB : 1], E[2][W::REM ? FB : 1];
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int f = 0; f < FB; ++f) acc[a][f] = float16v{};
+
+  W w[FB];
+  auto take_w = [&](uint32_t it, int un) {
+    const uint32_t bo = blk(it, ks) * W::BB;
+#pragma unroll
+    for (int f = 0; f < FB; ++f) w[f].take(wreg + f * L::WR, un, j, h, (wrow[f] + bo) & 2u);
+    // every read of the region has returned before the next loads into it go out
+    __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  };
+
+  half8 A[2][2];   // [part][tile]: the present step's until its instructions are issued, then the next one's
+  auto read_a = [&](int q, uint32_t g, uint32_t i) {
+    const uint8_t *p = xl + (g & 1u) * L::XG + i * 4096u + 256 * q;
+#pragma unroll
+    for (int a = 0; a < 2; ++a) A[q][a] = *(const half8 *)(p + 2048 * a);
+    __asm__ volatile("" ::: "memory");
+  };
+  half8 B[2][FB], R[2][W::REM ? FB : 1];
+  auto decode = [&](uint32_t set, uint32_t s) {
+#pragma unroll
+    for (int f = 0; f < FB; ++f) {
+      if constexpr (W::REM) B[set][f] = w[f].step2((int)(s % SU), R[set][f]);
+      else B[set][f] = w[f].step((int)s, h, lds);
+    }
+  };
+  auto low = [&](uint32_t set) {
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int f = 0; f < FB; ++f) {
+        float16v &d = W::SEP ? D2[a][W::SEP ? f : 0] : D[a][f];
+        d = mma(A[1][a], B[set][f], d);
+      }
+  };
+  auto high = [&](uint32_t set) {
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int f = 0; f < FB; ++f) D[a][f] = mma(A[0][a], B[set][f], D[a][f]);
+    if constexpr (W::REM) {
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int f = 0; f < FB; ++f) D2[a][f] = mma(A[0][a], R[set][f], D2[a][f]);
+    }
+  };
+  // D at the start of a block: the minima's sums, scaled, and the centres'
+  float dcur[FB];
+  auto open = [&]() {
+    if constexpr (MINS) {
+      const uint8_t *ml = lds + L::M0 + ks * 4096u + (j >> 4) * 1024u + 16u * ((W::MSTEP == 1u ? 16u : 32u) * h + (j & 15u));
+      half8 ms[2][W::MSTEP];
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (uint32_t q = 0; q < W::MSTEP; ++q) ms[a][q] = *(const half8 *)(ml + 2048 * a + 256u * q);
+#pragma unroll
+      for (int f = 0; f < FB; ++f) {
+        const half8 mb = w[f].mins(h), cb = w[f].centre(h);
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+          D[a][f] = float16v{};
+#pragma unroll
+          for (int q = (int)W::MSTEP - 1; q >= 0; --q) D[a][f] = mma(ms[a][q], mb, D[a][f]);
+#pragma unroll
+          for (int v = 0; v < 16; ++v) D[a][f][v] *= w[f].ratio;
+#pragma unroll
+          for (int q = (int)W::MSTEP - 1; q >= 0; --q) D[a][f] = mma(ms[a][q], cb, D[a][f]);
+        }
+      }
+    } else {
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int f = 0; f < FB; ++f) D[a][f] = float16v{};
+    }
+    if constexpr (W::SEP) {
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int f = 0; f < FB; ++f) D2[a][f] = float16v{};
+    }
+#pragma unroll
+    for (int f = 0; f < FB; ++f) dcur[f] = w[f].d;
+  };
+
+  // prologue: the first unit's weights, the first block's sums and scales, x of
+  // the first two groups
+  fetch_w(0u, 0);
+  fetch_m(0u);
+  fetch_x(0u, 0u);
+  fetch_x(0u, 1u);
+  wait_vm<XI>();
+  __syncthreads();
+  take_w(0u, 0);
+  fetch_w(W::UNITS == 1u ? 1u : 0u, W::UNITS == 1u ? 0 : 1);
+  read_a(1, 0u, 0u);
+  read_a(0, 0u, 0u);
+  decode(0u, 0u);
+
+  for (uint32_t it = 0; it < iters; ++it) {
+    open();
+#pragma unroll
+    for (uint32_t s = 0; s < 16u; ++s) {
+      const uint32_t cur = s & 1u, nxt = cur ^ 1u, g = s >> 2, gn = (g + ((s & 3u) == 3u)) & 3u, sn = (s + 1u) & 3u;
+      // lo parts; at a group's end, between the two, the next group's x is in
+      // LDS once every wave's own loads of it are (a group ago; the weights of
+      // the next unit went out after them), and the present group's buffer is
+      // free once every wave has read it
+      if constexpr (W::REM)
+        if (s == 8u) {
+#pragma unroll
+          for (int a = 0; a < 2; ++a)
+#pragma unroll
+            for (int f = 0; f < FB; ++f) {
+              E[a][f] = D[a][f];
+              D[a][f] = float16v{};
+            }
+        }
+      low(cur);
+      if ((s & 3u) == 3u) {
+        __builtin_amdgcn_sched_barrier(0);
+        if (g % (W::UNITS == 1u ? 4u : 2u) == 0u) wait_vm_lds<WI>();
+        else wait_vm_lds<0>();
+        __builtin_amdgcn_s_barrier();
+        __asm__ volatile("" ::: "memory");
+        if (g == 2u) fetch_m(it + 1u);
+        fetch_x(g < 2u ? it : it + 1u, (g + 2u) & 3u);
+      }
+      read_a(1, gn, sn);
+      if ((s + 1u) % SU == 0u) {
+        // the next unit: its weights into registers, and the loads of the one after
+        const uint32_t ni = s == 15u ? it + 1u : it;
+        const int un = s == 15u ? 0 : 1;
+        take_w(ni, un);
+        fetch_w(un + 1 == (int)W::UNITS ? ni + 1u : ni, un + 1 == (int)W::UNITS ? 0 : un + 1);
+      }
+      // hi parts, while the next step's weights are decoded
+      decode(nxt, (s + 1u) & 15u);
+      high(cur);
+#pragma unroll
+      for (int i = 0; i < 4 * FB; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
+      }
+      read_a(0, gn, sn);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // the fold
+    if (bl + 2u * it + ks < bh) {
+      const uint8_t *pp = lds + L::P0 + (it & 1u) * 512u + ks * 256u + 16u * h;
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const float4 p = *(const float4 *)(pp + 128 * a + 32 * g);
+#pragma unroll
+          for (int f = 0; f < FB; ++f)
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+              float t = D[a][f][4 * g + v];
+              if constexpr (W::REM) t = E[a][f][4 * g + v] + t;
+              if constexpr (W::SEP) t += D2[a][f][4 * g + v];
+              acc[a][f][4 * g + v] =
+                  __builtin_fmaf(t * dcur[f], v == 0 ? p.x : v == 1 ? p.y : v == 2 ? p.z : p.w, acc[a][f][4 * g + v]);
+            }
+        }
+    }
+  }
+  wait_vm<0>();
+  __syncthreads();
+
+  // the two k slices' sums, slice 0 + slice 1: a wave writes 32 FB tokens x 32
+  // rows of its row group (two row tiles: tile ks, one: token tile ks) and hands
+  // the rest over in LDS
+  float *const red = (float *)lds;
+  float16v sum[FB];
+#pragma unroll
+  for (int i = 0; i < FB; ++i)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+      const float a0 = acc[i][0][v], a1 = FB == 2 ? acc[i][FB - 1][v] : acc[1][0][v];
+      sum[i][v] = ks ? a1 : a0;
+      red[((wave * FB + i) * 16u + v) * 64u + lane] = ks ? a0 : a1;
+    }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < FB; ++i)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) sum[i][v] += red[(((wave ^ 4u) * FB + i) * 16u + v) * 64u + lane];
+
+  if (ksl > 1u) {
+    // k slices over workgroups, as in eff_gemm_sx.hip: the last of the tile's
+    // ksl workgroups to arrive adds the slices in slice order
+    constexpr int kSc1 = 16;   // cache policy bit 4: sc1
+    constexpr uint32_t NE = kTokTile * sxt_rows<TYPE>();
+    uint32_t *const arrived = (uint32_t *)(lds + L::BYTES - 16u);
+    const rsrc_t prs = make_rsrc(part + (uint64_t)lin * ksl * NE, (uint64_t)ksl * NE * 4u);
+    auto off = [&](uint32_t zz, uint32_t a, uint32_t v4) {
+      return (int)(zz * (NE * 4u) + (((wave * FB + a) * 4u + v4) * 64u + lane) * 16u);
+    };
+#pragma unroll
+    for (uint32_t a = 0; a < (uint32_t)FB; ++a)
+#pragma unroll
+      for (uint32_t v = 0; v < 4u; ++v) {
+        const u32x4 o = {__float_as_uint(sum[a][4 * v]), __float_as_uint(sum[a][4 * v + 1]),
+                         __float_as_uint(sum[a][4 * v + 2]), __float_as_uint(sum[a][4 * v + 3])};
+        __builtin_amdgcn_raw_buffer_store_b128(o, prs, off(z, a, v), 0, kSc1);
+      }
+    __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();   // every wave's sums are stored
+    if (tid == 0u) *arrived = __hip_atomic_fetch_add(cnt + lin, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (*arrived != ksl - 1u) return;
+    if (tid == 0u) __hip_atomic_store(cnt + lin, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (uint32_t zz = 0; zz < ksl; ++zz) {
+#pragma unroll
+      for (uint32_t a = 0; a < (uint32_t)FB; ++a)
+#pragma unroll
+        for (uint32_t v = 0; v < 4u; ++v) {
+          const u32x4 o = __builtin_amdgcn_raw_buffer_load_b128(prs, off(zz, a, v), 0, kSc1);
+#pragma unroll
+          for (int c = 0; c < 4; ++c)
+            sum[a][4 * v + c] = zz ? sum[a][4 * v + c] + __uint_as_float(o[c]) : __uint_as_float(o[c]);
+        }
+    }
+  }
+  const uint32_t row = r0 + (FB == 2 ? 32u * ks : 0u) + j;
+  if (row >= rows) return;
+#pragma unroll
+  for (uint32_t a = 0; a < (uint32_t)FB; ++a)
+#pragma unroll
+    for (uint32_t v = 0; v < 16u; ++v) {
+      const uint32_t tok = kTokTile * tt0 + 32u * (FB == 2 ? a : ks) + 8u * (v >> 2) + 4u * h + (v & 3u);
+      if (tok < tokens) y[(uint64_t)tok * rows + row] = sum[a][v];
+    }
+}
+
+struct SxtPlan {
+  uint32_t row_tiles, tok_tiles, ksl;
+};
+
+SxtPlan sxt_plan(const WeightView &wv, uint32_t tokens, uint32_t ksl) {
+  return {(wv.rows + sxt_row_tile(wv.type) - 1u) / sxt_row_tile(wv.type), (tokens + kTokTile - 1u) / kTokTile,
+          (uint32_t)max(1u, min(ksl, wv.k / 256u))};
+}
+
+template <int TYPE>
+hipError_t sxt_go(const WeightView &wv, const uint8_t *xa, const float *xp, uint32_t tiles, float *y,
+                  uint32_t tokens, const SxtPlan &p, void *sk, hipStream_t s) {
+  const uint64_t nb = wv.k / 256u, xb = (uint64_t)tiles * nb * sx_slots<TYPE>() * 1024u;
+  if (tiles < 4u * p.tok_tiles || xb >= (1ull << 32)) return hipErrorInvalidValue;
+  if (p.ksl > 1u && (!sk || (uint64_t)p.row_tiles * p.tok_tiles > kSliceCntBytes / 4u)) return hipErrorInvalidValue;
+  uint32_t *cnt = (uint32_t *)sk;
+  float *part = sk ? (float *)((uint8_t *)sk + kSliceCntBytes) : nullptr;
+  hipLaunchKernelGGL((k_sxt<TYPE>), dim3(p.row_tiles * p.tok_tiles * p.ksl), dim3(512), 0, s, wv, xa, xp, y,
+                     tokens, (uint32_t)xb, (uint32_t)(tiles * nb * 64u), p.row_tiles, p.tok_tiles, p.ksl, part, cnt);
+  return hipGetLastError();
+}
+
+}  // namespace
+
+size_t sxt_sk_bytes(const WeightView &wv, uint32_t tokens, uint32_t ksl) {
+  const SxtPlan p = sxt_plan(wv, tokens, ksl);
+  if (p.ksl < 2u) return 0;
+  return kSliceCntBytes + (size_t)p.row_tiles * p.tok_tiles * p.ksl * (kTokTile * sxt_row_tile(wv.type) * 4u);
+}
+
+hipError_t launch_sxt(const WeightView &wv, const void *xa, const void *xp, uint32_t tiles, float *y,
+                      uint32_t tokens, uint32_t ksl, void *sk, hipStream_t s) {
+  const SxtPlan p = sxt_plan(wv, tokens, ksl);
+  const uint8_t *a = (const uint8_t *)xa;
+  const float *b = (const float *)xp;
+  switch (wv.type) {
+    case Q4_K: return sxt_go<Q4_K>(wv, a, b, tiles, y, tokens, p, sk, s);
+    case Q6_K: return sxt_go<Q6_K>(wv, a, b, tiles, y, tokens, p, sk, s);
+    case Q2_K: return sxt_go<Q2_K>(wv, a, b, tiles, y, tokens, p, sk, s);
+    case IQ2_XXS: return sxt_go<IQ2_XXS>(wv, a, b, tiles, y, tokens, p, sk, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+}  // namespace eff

@@ -1,0 +1,97 @@
+"""The split-x product over LDS-shared tiles (prompts of Q4_K, Q2_K, Q6_K and
+IQ2_XXS) against the f64 product of the oracle's weights, at the edges of its
+tiles: rows and tokens past whole tiles, one block of k, odd block counts (one k
+slice of the workgroup then ends early), k slices over workgroups, blocks whose
+scale is zero, and non-finite x."""
+import numpy as np
+import pytest
+
+from test_gpu_parity import make_weights
+
+pytestmark = pytest.mark.gpu
+
+# x is kept to 2^-22 of each value, and a sum is at most 40 roundings to f32 per
+# block of 256 and one per block and slice; rounding errors of random sign over
+# them stay under 16 ulp (2^-20) of the output's norm
+REL = 2.0 ** -20
+
+# (type, rows, k, tokens): shapes at which the planner takes the shared tiles,
+# alone (the first of each type) and in 2 to 8 k slices
+SHAPES = [("Q4_K", 513, 256, 4000), ("Q4_K", 1000, 4352, 520), ("Q4_K", 513, 8192, 449),
+          ("Q2_K", 513, 256, 4000), ("Q2_K", 1000, 8192, 130),
+          ("Q6_K", 1000, 256, 520), ("Q6_K", 777, 768, 1000), ("Q6_K", 513, 2304, 1000), ("Q6_K", 1000, 8192, 65),
+          ("IQ2_XXS", 777, 256, 2000), ("IQ2_XXS", 513, 4352, 449)]
+
+
+def product(orc, tname, gguf, n, x, rows, k):
+    w = orc.dequant(orc.NAMES[tname], gguf, n).astype(np.float64).reshape(rows, k)
+    return x.astype(np.float64).reshape(-1, k) @ w.T
+
+
+def run(ctx, t, wb, x, rows, k, tokens):
+    xb, yb = ctx.upload(x), ctx.alloc(tokens * rows * 4)
+    ctx.qmatmul(t, wb, xb, yb, rows, k, tokens)
+    y = yb.read(np.float32).reshape(tokens, rows)
+    ctx.qmatmul(t, wb, xb, yb, rows, k, tokens)
+    again = yb.read(np.float32).reshape(tokens, rows)
+    xb.free(); yb.free()
+    assert np.array_equal(y.view(np.uint32), again.view(np.uint32))   # whatever the order of arrival
+    return y
+
+
+@pytest.mark.parametrize("tname,rows,k,tokens", SHAPES)
+def test_shared_tiles_vs_f64(ctx, eff, orc, tname, rows, k, tokens):
+    t, data, gguf, n = make_weights(eff, tname, rows, k, 71)
+    x = eff.fill_normal(72, 1.0, tokens * k)
+    if tname in ("Q4_K", "Q2_K"):   # every fifth block: scale 0, its minima stay
+        b = data.reshape(n, -1)
+        b[::5, (0, 1) if tname == "Q4_K" else (80, 81)] = 0
+    wb = ctx.upload(data)
+    y = run(ctx, t, wb, x, rows, k, tokens)
+    ref = product(orc, tname, gguf, n, x, rows, k)
+    rel = np.linalg.norm(y - ref) / np.linalg.norm(ref)
+    print(f"shared tiles {tname} {rows}x{k} M={tokens}: rel_l2={rel:.2e}", flush=True)
+    assert rel <= REL
+    # no row or token is off by itself (a tile's edge)
+    err, scale = np.abs(y - ref), np.sqrt(np.mean(ref * ref))
+    assert err.max() <= 16 * REL * scale
+    # a forced configuration runs the other kernel: other sums, the same product
+    try:
+        ctx.set_option(eff.OPT_SPLIT_CONFIG, 1)
+        other = run(ctx, t, wb, x, rows, k, tokens)
+    finally:
+        ctx.set_option(eff.OPT_SPLIT_CONFIG, 0)
+    if k > 256:   # (over one block IQ2_XXS is summed alike)
+        assert not np.array_equal(y.view(np.uint32), other.view(np.uint32))
+    assert np.linalg.norm(other - ref) <= REL * np.linalg.norm(ref)
+    # prepared x: the same bits
+    nb, _ = ctx.qmatmul_x_layout(t, rows, k, tokens)
+    xb, xp, yb = ctx.upload(x), ctx.alloc(nb), ctx.alloc(tokens * rows * 4)
+    ctx.qmatmul_prepare_x(t, xb, xp, rows, k, tokens)
+    ctx.qmatmul_prepared(t, wb, xp, yb, rows, k, tokens)
+    assert np.array_equal(yb.read(np.uint32), y.view(np.uint32).ravel())
+    for b in (wb, xb, xp, yb):
+        b.free()
+
+
+@pytest.mark.parametrize("tname,rows,k,tokens", [SHAPES[1], SHAPES[6], SHAPES[10]])
+def test_shared_tiles_range_and_non_finite(ctx, eff, orc, tname, rows, k, tokens):
+    """x of mixed magnitudes (blocks of 1e-20 to 1e20), and tokens holding an
+    infinity or a NaN, whose outputs become non-finite and no other's."""
+    t, data, gguf, n = make_weights(eff, tname, rows, k, 81)
+    x = eff.fill_normal(82, 1.0, tokens * k).reshape(tokens, k)
+    x[0:4] *= 1e-20
+    x[4:8] *= 1e20
+    x[70, :256] *= 1e-3
+    x[70, 300 % k] *= 1e4
+    bad = x.copy()
+    bad[9, 5], bad[tokens - 1, k - 1] = np.inf, np.nan
+    wb = ctx.upload(data)
+    y = run(ctx, t, wb, bad, rows, k, tokens)
+    ref = product(orc, tname, gguf, n, x, rows, k)
+    good = np.ones(tokens, bool)
+    good[[9, tokens - 1]] = False
+    assert not np.isfinite(y[~good]).any() and np.isfinite(y[good]).all()
+    rel = np.linalg.norm(y - ref, axis=1)[good] / np.linalg.norm(ref, axis=1)[good]
+    assert rel.max() <= 2 * REL
+    wb.free()
