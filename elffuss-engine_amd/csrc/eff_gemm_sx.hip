@@ -522,7 +522,7 @@ __global__ __launch_bounds__(NW * 64) void k_sx(WeightView wv, const uint8_t *__
   // offsets per lane: 3 steps ahead at 4 token tiles keep it within the VGPRs;
   // the types folded per group of steps hold more state: fewer steps ahead)
   constexpr bool MS = W::FG < 16;
-  constexpr uint32_t P = TT == 1 ? 16u : TT == 2 ? (MS ? 4u : 8u) : TYPE == Q4_K ? 3u : MS ? 2u : 4u;
+  constexpr uint32_t P = TT == 1 ? 16u : TT == 2 ? (MS ? 4u : 8u) : TT == 3 ? (RF == 1 ? 4u : 5u) : TYPE == Q4_K ? 3u : MS ? 2u : 4u;
   constexpr uint32_t ROWS = L::ROWS, ND = L::ND;
   __shared__ __align__(16) uint8_t lds_s[FX ? 16u : L::BYTES];
   extern __shared__ __align__(16) uint8_t lds_d[];
@@ -820,12 +820,17 @@ struct SxPlan {
 };
 
 // The types folded per group of steps (Q8_0, Q8_0R, Q6_K) take at most 2
-// token tiles per wave: with 4 their folds' state does not fit the registers.
+// token tiles per wave: with more their folds' state does not fit the registers.
 uint32_t sx_tt_max(int type) { return type == Q8_0 || type == Q8_0R || type == Q6_K ? 2u : 4u; }
 
+// Three tiles per wave where that leaves fewer tiles of padding than four (33-48
+// tokens: 3 tiles instead of 4; 65-96: 6 instead of 8; the same bits; us, four
+// tiles / three: Q4_K 14336 x 4096 at 33 tokens 32.8 / 28.8, 8192 x 2048 at 96
+// 20.1 / 17.4; Q2_K 19.8 / 15.7, at 48 12.4 / 10.3; IQ2_XXS 14336 x 4096 at 40
+// 34.1 / 28.0).
 void sx_tiles(int type, uint32_t tokens, uint32_t &tt, uint32_t &groups) {
   const uint32_t ttn = (tokens + 15u) / 16u;
-  tt = ttn <= 1u ? 1u : ttn <= 2u || sx_tt_max(type) == 2u ? 2u : 4u;
+  tt = ttn <= 1u ? 1u : ttn <= 2u || sx_tt_max(type) == 2u ? 2u : (ttn + 2u) / 3u * 3u < (ttn + 3u) / 4u * 4u ? 3u : 4u;
   groups = (ttn + tt - 1u) / tt;
 }
 
@@ -988,6 +993,9 @@ hipError_t sx_main(const WeightView &wv, const uint8_t *xa, uint32_t tiles, floa
   switch (p.tt) {
     case 1: return sx_cfg<TYPE, 1>(wv, xa, xp, y, tokens, p, sk, s);
     case 2: return sx_cfg<TYPE, 2>(wv, xa, xp, y, tokens, p, sk, s);
+    case 3:
+      if constexpr (SxW<TYPE>::FG == 16) return sx_cfg<TYPE, 3>(wv, xa, xp, y, tokens, p, sk, s);
+      return hipErrorInvalidValue;   // not planned (sx_tt_max)
     default:
       if constexpr (SxW<TYPE>::FG == 16) return sx_cfg<TYPE, 4>(wv, xa, xp, y, tokens, p, sk, s);
       return hipErrorInvalidValue;   // not planned (sx_tt_max)

@@ -17,10 +17,10 @@ REL = 2.0 ** -20
 
 # (type, rows, k, tokens): shapes at which the planner takes the shared tiles,
 # alone (the first of each type) and in 2 to 8 k slices
-SHAPES = [("Q4_K", 513, 256, 4000), ("Q4_K", 1000, 4352, 520), ("Q4_K", 513, 8192, 449),
-          ("Q2_K", 513, 256, 4000), ("Q2_K", 1000, 8192, 130),
+SHAPES = [("Q4_K", 513, 256, 4000), ("Q4_K", 1000, 4352, 1000), ("Q4_K", 513, 8192, 501),
+          ("Q2_K", 513, 256, 4000), ("Q2_K", 513, 8192, 501),
           ("Q6_K", 1000, 256, 520), ("Q6_K", 777, 768, 1000), ("Q6_K", 513, 2304, 1000), ("Q6_K", 1000, 8192, 65),
-          ("IQ2_XXS", 777, 256, 2000), ("IQ2_XXS", 513, 4352, 449)]
+          ("IQ2_XXS", 777, 256, 2000), ("IQ2_XXS", 513, 4352, 501)]
 
 
 def product(orc, tname, gguf, n, x, rows, k):
@@ -94,4 +94,32 @@ def test_shared_tiles_range_and_non_finite(ctx, eff, orc, tname, rows, k, tokens
     assert not np.isfinite(y[~good]).any() and np.isfinite(y[good]).all()
     rel = np.linalg.norm(y - ref, axis=1)[good] / np.linalg.norm(ref, axis=1)[good]
     assert rel.max() <= 2 * REL
+    wb.free()
+
+
+@pytest.mark.parametrize("tname", ["Q4_K", "Q2_K", "IQ2_XXS"])
+@pytest.mark.parametrize("tokens", [33, 48, 65, 96, 129])
+def test_three_token_tiles(ctx, eff, orc, tname, tokens):
+    """Token counts that three tiles of 16 per wave fit better than four (33-48,
+    65-96, 129-144), in both workgroup shapes and from a prepared x."""
+    rows, k = 77, 1280
+    t, data, gguf, n = make_weights(eff, tname, rows, k, 91)
+    x = eff.fill_normal(92, 1.0, tokens * k)
+    ref = product(orc, tname, gguf, n, x, rows, k)
+    wb = ctx.upload(data)
+    try:
+        for cfg in (0, 1, 2):
+            ctx.set_option(eff.OPT_SPLIT_CONFIG, cfg)
+            y = run(ctx, t, wb, x, rows, k, tokens)
+            assert np.linalg.norm(y - ref) <= REL * np.linalg.norm(ref), cfg
+            assert np.abs(y - ref).max() <= 16 * REL * np.sqrt(np.mean(ref * ref)), cfg
+            nb, _ = ctx.qmatmul_x_layout(t, rows, k, tokens)
+            xb, xp, yb = ctx.upload(x), ctx.alloc(nb), ctx.alloc(tokens * rows * 4)
+            ctx.qmatmul_prepare_x(t, xb, xp, rows, k, tokens)
+            ctx.qmatmul_prepared(t, wb, xp, yb, rows, k, tokens)
+            assert np.array_equal(yb.read(np.uint32), y.view(np.uint32).ravel())
+            for b in (xb, xp, yb):
+                b.free()
+    finally:
+        ctx.set_option(eff.OPT_SPLIT_CONFIG, 0)
     wb.free()
