@@ -73,3 +73,27 @@ def test_gather_errors(ctx, eff):
     with pytest.raises(eff.EffError) as e:
         ctx.gather(eff.Q8_0R, rb, ib, out, dim, 1)          # unmarked repacked buffer
     assert e.value.code == eff.E_MARK
+
+
+@pytest.mark.parametrize("tname,dim,tokens", [("Q8_0", 32, 3), ("Q8_0R", 96, 1), ("Q8_0", 1056, 5), ("Q6_K", 768, 2),
+                                              ("Q4_K", 4352, 7), ("Q8_0", 32768, 2), ("Q2_K", 32768, 1)])
+def test_gather_norm_dims(ctx, eff, orc, tname, dim, tokens):
+    """Rows shorter than a workgroup's 1024 columns, not a multiple of them, and
+    the longest. x is bit-identical to the decoder; nrm is off by the roundings of its sum (dim / 256 + 8 f32 additions
+    of squares, halved by the root) and of three operations."""
+    rows, eps = 40, 1e-6
+    t, data, gguf, n = make_weights(eff, tname, rows, dim, 610 + dim)
+    ids = np.random.default_rng(dim).integers(0, rows, tokens).astype(np.uint32)
+    wn = eff.fill_normal(611, 1.0, dim)
+    wb, ib, wnb = upload_w(ctx, eff, tname, data, n), ctx.upload(ids), ctx.upload(wn)
+    x, nrm = ctx.alloc(tokens * dim * 4), ctx.alloc(tokens * dim * 4)
+    ctx.gather_norm(t, wb, ib, wnb, eps, x, nrm, dim, tokens)
+    rows_f = oracle_rows(eff, orc, tname, gguf, n, dim, ids)
+    assert np.array_equal(x.read(np.uint32).reshape(tokens, dim), rows_f.view(np.uint32))
+    r64 = rows_f.astype(np.float64)
+    want = r64 / np.sqrt((r64 * r64).mean(axis=1, keepdims=True) + eps) * wn.astype(np.float64)[None, :]
+    got = nrm.read(np.float32).reshape(tokens, dim).astype(np.float64)
+    tol = (0.5 * (dim / 256 + 8) + 3) * 2.0 ** -24
+    assert np.max(np.abs(got - want) / np.maximum(np.abs(want), 1e-30)) <= tol
+    for b in (wb, ib, wnb, x, nrm):
+        b.free()
