@@ -501,11 +501,13 @@ struct SxLds {
 // f32 xf: per wave, block by block, x's rows go to LDS by direct-to-LDS loads
 // issued before the block's weights, so that the preparation runs while the
 // weights are in flight. LDS (dynamic): the tables and stages as without FX,
-// then per wave sx_fx_bytes<TYPE>(): 8 x 1 KB of raw x, NS fragment slots of
-// kSxFxSlot bytes, 16 scales.
+// then per wave sx_fx_bytes<TYPE>(): NS fragment slots of kSxFxSlot bytes, which
+// take the place of the block's 8 x 1 KB of raw x once that is in registers, and
+// 16 scales.
 template <int TYPE>
 constexpr uint32_t sx_fx_bytes() {
-  return 8u * 1024u + sx_slots<TYPE>() * kSxFxSlot + 64u;
+  static_assert(sx_slots<TYPE>() * kSxFxSlot >= 8u * 1024u, "raw x");
+  return sx_slots<TYPE>() * kSxFxSlot + 64u;
 }
 
 template <int TYPE, int TT, int RF, int NW, bool FX>
@@ -576,7 +578,7 @@ __global__ __launch_bounds__(NW * 64) void k_sx(WeightView wv, const uint8_t *__
   const rsrc_t xsrc = make_rsrc(xa, xa_bytes);
   // FX: this wave's raw x, fragments and scales
   uint8_t *const xw = lds + L::TAB + L::WORK + wave * sx_fx_bytes<TYPE>();
-  uint8_t *const xfr = xw + 8u * 1024u;
+  uint8_t *const xfr = xw;
   float *const xps = (float *)(xfr + NS * kSxFxSlot);
   const rsrc_t fsrc = make_rsrc(xf, (uint64_t)tokens * wv.k * 4u);
   // the lane's fragment row: lanes of tokens 8..15 read the row of token
@@ -584,8 +586,8 @@ __global__ __launch_bounds__(NW * 64) void k_sx(WeightView wv, const uint8_t *__
   // never written), so that every read is unmasked and can be issued early
   const uint32_t frow = 16u * (lane >> 5) + 8u * ((lane >> 4) & 1u) + (lane & 7u);
   if constexpr (FX) {
-    // the rows of tokens past `tokens` and their scales stay zero
-    for (uint32_t o = 16u * lane; o < NS * kSxFxSlot + 64u; o += 1024u) *(u32x4 *)(xfr + o) = u32x4{0u, 0u, 0u, 0u};
+    // the scales of tokens 8..15 stay zero
+    if (lane < 16u) xps[lane] = 0.f;
   }
 
   float acc[TT][RF][8];
@@ -767,7 +769,7 @@ __global__ __launch_bounds__(NW * 64) void k_sx(WeightView wv, const uint8_t *__
 #pragma unroll
     for (uint32_t w = 0; w < (uint32_t)NW; ++w) sum[i] += red[w * L::NE + tid + NT * i];
   }
-  if (!FX && ksl > 1u) {
+  if (ksl > 1u) {
     // k slices: each workgroup of the tile stores its sums; the last of the
     // tile's ksl workgroups to arrive adds the slices in slice order, ((s0 +
     // s1) + s2) ..., which does not depend on the order of arrival, and
@@ -952,15 +954,19 @@ hipError_t sx_go(const WeightView &wv, const uint8_t *xa, const float *xp, float
 
 // The product with its own preparation (up to 8 tokens, 32 rows x 8 waves).
 template <int TYPE>
-hipError_t sx_go_fx(const WeightView &wv, const float *x, float *y, uint32_t tokens, const SxPlan &p, hipStream_t s) {
+hipError_t sx_go_fx(const WeightView &wv, const float *x, float *y, uint32_t tokens, const SxPlan &p, void *sk,
+                    hipStream_t s) {
   using L = SxLds<TYPE, 1, 1, 8>;
   constexpr uint32_t lds = L::TAB + L::WORK + 8u * sx_fx_bytes<TYPE>();
   static_assert(lds + 16u <= kMxMaxLds, "fused split-x LDS");
+  if (p.ksl > 1u && (!sk || p.row_tiles > kSliceCntBytes / 4u)) return hipErrorInvalidValue;
+  uint32_t *cnt = (uint32_t *)sk;
+  float *part = sk ? (float *)((uint8_t *)sk + kSliceCntBytes) : nullptr;
   static std::atomic<uint64_t> attr{0};
   const hipError_t e = lds_limit_once((const void *)k_sx<TYPE, 1, 1, 8, true>, (int)lds, attr);
   if (e != hipSuccess) return e;
-  hipLaunchKernelGGL((k_sx<TYPE, 1, 1, 8, true>), dim3(p.row_tiles, 1), dim3(8 * 64), lds, s, wv, nullptr, nullptr,
-                     y, tokens, p.nbw, 0u, x, 1u, nullptr, nullptr);
+  hipLaunchKernelGGL((k_sx<TYPE, 1, 1, 8, true>), dim3(p.row_tiles * p.ksl, 1), dim3(8 * 64), lds, s, wv, nullptr,
+                     nullptr, y, tokens, p.nbw, 0u, x, p.ksl, part, cnt);
   return hipGetLastError();
 }
 
@@ -981,6 +987,17 @@ hipError_t sx_cfg(const WeightView &wv, const uint8_t *xa, const float *xp, floa
 bool sx_fx(int type, uint32_t tokens, int cfg, const SxPlan &p, uint32_t k) {
   return (type == Q2_K || type == IQ2_XXS) && cfg == 0 && tokens <= 8u && p.cfg == 0u && p.ksl == 1u &&
          (uint64_t)p.row_tiles * p.groups * k <= 256ull * 2048u;
+}
+
+// Q8_0, Q8_0R and Q6_K take the one launch too where the call brings x itself
+// (their prepared-x calls stay, with the same bits), also in k slices, whose
+// workgroups prepare their slice's blocks only (us, two launches / one, 8 tokens:
+// Q8_0 2048 x 8192 12.6 / 11.5, Q6_K 13.0 / 11.9, Q8_0 1024 x 8192 11.6 / 10.3,
+// 4096 x 4608 12.8 / 11.8; beyond 256 x 2304: Q8_0R 4096 x 5120 13.1 / 14.6,
+// Q8_0 5120 x 5120 20.9 / 24.5, 4096 x 14336 22.8 / 25.3).
+bool sx_fx_plain(int type, uint32_t tokens, int cfg, const SxPlan &p, uint32_t k) {
+  return (type == Q8_0 || type == Q8_0R || type == Q6_K) && cfg == 0 && tokens <= 8u && p.cfg == 0u && !p.shared &&
+         (uint64_t)p.row_tiles * p.groups * k <= 256ull * 2304u;
 }
 
 // The product from x prepared in `xa` for `tiles` token tiles (at least the
@@ -1007,7 +1024,9 @@ hipError_t sx_type(const WeightView &wv, const float *x, float *y, uint32_t toke
                    uint32_t ksl_opt, void *sk, hipStream_t s) {
   const SxPlan p = sx_plan(wv, tokens, cfg, ksl_opt);
   if constexpr (TYPE == Q2_K || TYPE == IQ2_XXS)
-    if (sx_fx(TYPE, tokens, cfg, p, wv.k)) return sx_go_fx<TYPE>(wv, x, y, tokens, p, s);
+    if (sx_fx(TYPE, tokens, cfg, p, wv.k)) return sx_go_fx<TYPE>(wv, x, y, tokens, p, nullptr, s);
+  if constexpr (TYPE == Q8_0 || TYPE == Q8_0R || TYPE == Q6_K)
+    if (sx_fx_plain(TYPE, tokens, cfg, p, wv.k)) return sx_go_fx<TYPE>(wv, x, y, tokens, p, sk, s);
   const uint32_t tiles = sx_tile_count(TYPE, tokens), nb = wv.k / 256u;   // blocks of 256 weights
   uint8_t *xa = scratch;
   float *xp = (float *)(scratch + (uint64_t)tiles * nb * sx_slots<TYPE>() * 1024u);

@@ -6,7 +6,7 @@ scale is zero, and non-finite x."""
 import numpy as np
 import pytest
 
-from test_gpu_parity import make_weights
+from test_gpu_parity import make_weights, upload_w
 
 pytestmark = pytest.mark.gpu
 
@@ -123,3 +123,27 @@ def test_three_token_tiles(ctx, eff, orc, tname, tokens):
     finally:
         ctx.set_option(eff.OPT_SPLIT_CONFIG, 0)
     wb.free()
+
+
+@pytest.mark.parametrize("tname", ["Q8_0", "Q8_0R", "Q6_K"])
+@pytest.mark.parametrize("rows,k,tokens", [(2048, 8192, 8), (77, 8192, 7), (1000, 4608, 8), (130, 16384, 5)])
+def test_one_launch_in_k_slices(ctx, eff, orc, tname, rows, k, tokens):
+    """5-8 tokens where the int8 GEMVs do not run: x prepared inside the product
+    (whose workgroups take slices of k), with the bits of the two-launch form."""
+    t, data, gguf, n = make_weights(eff, tname, rows, k, 95)
+    x = eff.fill_normal(96, 1.0, tokens * k)
+    x[:256] *= 1e-3
+    x[k:k + 256] *= 1e6
+    wb = upload_w(ctx, eff, tname, data, n)
+    before = ctx.stats()["split"]
+    y = run(ctx, t, wb, x, rows, k, tokens)
+    assert ctx.stats()["split"] == before + 2
+    ref = product(orc, "Q8_0" if tname == "Q8_0R" else tname, gguf, n, x, rows, k)
+    assert (np.linalg.norm(y - ref, axis=1) <= REL * np.linalg.norm(ref, axis=1)).all()
+    nb, _ = ctx.qmatmul_x_layout(t, rows, k, tokens)
+    xb, xp, yb = ctx.upload(x), ctx.alloc(nb), ctx.alloc(tokens * rows * 4)
+    ctx.qmatmul_prepare_x(t, xb, xp, rows, k, tokens)
+    ctx.qmatmul_prepared(t, wb, xp, yb, rows, k, tokens)
+    assert np.array_equal(yb.read(np.uint32), y.view(np.uint32).ravel())
+    for b in (wb, xb, xp, yb):
+        b.free()
