@@ -669,8 +669,12 @@ __global__ __launch_bounds__(NW * 64) void k_sx(WeightView wv, const uint8_t *__
     const uint32_t *rp[RF];
     // PRE: the weight dwords of all 16 steps in registers before the steps
     // (whose prefetch of x fragments keeps the compiler from hoisting LDS
-    // reads); the 4-tile kernels have no registers to spare
-    constexpr bool PRE = !FX && TT <= 2 && W::NP > 0;
+    // reads): up to 2 token tiles, and the 64-row waves (one per SIMD, with its
+    // 512 registers) of IQ2_XXS and Q2_K (us, LDS reads in the steps / registers:
+    // IQ2_XXS 8192 x 2048 at 128 tokens 21.5 / 20.0, 14336 x 4096 at 40 27.7 /
+    // 25.8, Q2_K 20.6 / 19.9; Q4_K's header then leaves the compiler moving
+    // registers, 14336 x 4096 at 33 28.8 / 43.0)
+    constexpr bool PRE = !FX && W::NP > 0 && (TT <= 2 || (RF == 2 && TYPE != Q4_K));
     uint32_t pr[RF][PRE ? W::NP : 1];
 #pragma unroll
     for (int f = 0; f < RF; ++f) {

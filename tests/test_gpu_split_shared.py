@@ -98,10 +98,10 @@ def test_shared_tiles_range_and_non_finite(ctx, eff, orc, tname, rows, k, tokens
 
 
 @pytest.mark.parametrize("tname", ["Q4_K", "Q2_K", "IQ2_XXS"])
-@pytest.mark.parametrize("tokens", [33, 48, 65, 96, 129])
+@pytest.mark.parametrize("tokens", [33, 48, 64, 65, 96, 129])
 def test_three_token_tiles(ctx, eff, orc, tname, tokens):
     """Token counts that three tiles of 16 per wave fit better than four (33-48,
-    65-96, 129-144), in both workgroup shapes and from a prepared x."""
+    65-96, 129-144; 64 takes four), in both workgroup shapes and from a prepared x."""
     rows, k = 77, 1280
     t, data, gguf, n = make_weights(eff, tname, rows, k, 91)
     x = eff.fill_normal(92, 1.0, tokens * k)
