@@ -357,15 +357,21 @@ __global__ __launch_bounds__(kNW * 64) void k_gemm_q8(WeightView wv, const _Floa
   uint32_t lane_e;
   __asm__ volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane_e));
   const uint32_t ne = lane_e & 31u, he = lane_e >> 5;
-  // outputs v = 4 q .. 4 q + 3 of fragment (fi, fj)
+  // outputs v = 4 q .. 4 q + 3 of fragment (fi, fj), past the caches: a tile's
+  // outputs all leave at the end of its workgroup, and what stays dirty in L2 is
+  // written back before the next launch starts (us with the x conversion, plain /
+  // nontemporal stores: 8192 x 2048 at 512 tokens 34.9 / 33.1, at 2048 86.5 / 84.5, 14336 x
+  // 4096 at 256 51.7 / 49.2, 1024 x 4096 at 1000 27.0 / 26.3; 2048 x 8192 at 64
+  // 20.7 / 20.7)
   auto put = [&](int fi, int fj, int q, float4 v) {
     const uint32_t row = n0 + kFN * 32u * wn + 32u * (uint32_t)fj + ne;
     const uint32_t tok = t0 + kFM * 32u * wm + 32u * (uint32_t)fi + 8u * (uint32_t)q + 4u * he;
     if (row >= rows) return;
-    if (tok < tokens) y[(uint64_t)tok * rows + row] = v.x;
-    if (tok + 1u < tokens) y[(uint64_t)(tok + 1u) * rows + row] = v.y;
-    if (tok + 2u < tokens) y[(uint64_t)(tok + 2u) * rows + row] = v.z;
-    if (tok + 3u < tokens) y[(uint64_t)(tok + 3u) * rows + row] = v.w;
+    float *o = y + (uint64_t)tok * rows + row;
+    if (tok < tokens) __builtin_nontemporal_store(v.x, o);
+    if (tok + 1u < tokens) __builtin_nontemporal_store(v.y, o + rows);
+    if (tok + 2u < tokens) __builtin_nontemporal_store(v.z, o + 2ull * rows);
+    if (tok + 3u < tokens) __builtin_nontemporal_store(v.w, o + 3ull * rows);
   };
   auto mine = [&](int fi, int fj, int q) {
     return make_float4(acc[fi][fj][4 * q], acc[fi][fj][4 * q + 1], acc[fi][fj][4 * q + 2], acc[fi][fj][4 * q + 3]);
