@@ -812,7 +812,7 @@ __global__ __launch_bounds__(NW * 64) void k_sx(WeightView wv, const uint8_t *__
     const uint32_t le = e & 63u, v = (e >> 6) & 7u, fr = e >> 9, f = fr % RF, tt = fr / RF;
     const uint32_t row = r0 + 32u * f + (le & 31u);
     const uint32_t tok = (tg * TT + tt) * 16u + 8u * (v >> 2) + 4u * (le >> 5) + (v & 3u);
-    if (row < rows && tok < tokens) y[(uint64_t)tok * rows + row] = sum[i];
+    if (row < rows && tok < tokens) __builtin_nontemporal_store(sum[i], y + (uint64_t)tok * rows + row);
   }
 }
 

@@ -495,9 +495,9 @@ __global__ __launch_bounds__(512) void k_sxt(WeightView wv, const uint8_t *__res
   fetch_w(0u, 0);
   fetch_m(0u);
   fetch_x(0u, 0u);
-  fetch_x(0u, 1u);
-  wait_vm<XI>();
+  wait_vm<0>();
   __syncthreads();
+  fetch_x(0u, 1u);
   take_w(0u, 0);
   fetch_w(W::UNITS == 1u ? 1u : 0u, W::UNITS == 1u ? 0 : 1);
   read_a(1, 0u, 0u);
@@ -638,7 +638,7 @@ __global__ __launch_bounds__(512) void k_sxt(WeightView wv, const uint8_t *__res
 #pragma unroll
     for (uint32_t v = 0; v < 16u; ++v) {
       const uint32_t tok = kTokTile * tt0 + 32u * (FB == 2 ? a : ks) + 8u * (v >> 2) + 4u * h + (v & 3u);
-      if (tok < tokens) y[(uint64_t)tok * rows + row] = sum[a][v];
+      if (tok < tokens) __builtin_nontemporal_store(sum[a][v], y + (uint64_t)tok * rows + row);
     }
 }
 
