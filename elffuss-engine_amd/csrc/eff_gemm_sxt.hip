@@ -8,10 +8,10 @@
 // clock and CU with the matrix cores busy, all that a CU's vector memory path
 // delivers. Here a workgroup's waves share x through LDS.
 //
-// Workgroup: 8 waves (2 per SIMD) over 64 tokens x 256 rows, as 4 groups of 64
-// rows x 2 slices of k (slice z takes every second block of 256). A wave holds
-// 2 x 2 tiles of 32 tokens x 32 rows: per step of 16 k it reads 2 lo and 2 hi
-// fragments of x (4 KB) for 8 v_mfma_f32_32x32x16_f16, decodes its 2 weight
+// Workgroup: 8 waves (2 per SIMD) over 64 tokens x 128 FB rows, as 4 groups of
+// 32 FB rows x 2 slices of k (slice z takes every second block of 256). A wave
+// holds 2 x FB tiles of 32 tokens x 32 rows: per step of 16 k it reads 2 lo and 2
+// hi fragments of x (4 KB) for 4 FB v_mfma_f32_32x32x16_f16, decodes its FB weight
 // fragments in registers, and adds lo and hi into one accumulator per tile,
 //   D += u lo, D += u hi,
 // folded once per block: acc += D d p (p: x's block scales). x flows in groups of 4 steps through two
@@ -26,7 +26,7 @@
 // and D opens with the group sums' terms, -(dmin / d) sum mn_g S_g + 8 (1.5)
 // sum sc_g S_g (1.9e-7 against 3.2e-7, 1.8e-7 against 2.1e-7). IQ2_XXS and Q6_K
 // keep the lo parts in accumulators of their own, which leaves registers for
-// one row tile per wave (1.3e-7 as before; Q6_K 1.2e-7 against 1.7e-7, its hi
+// one row tile per wave (FB = 1) (1.3e-7 as before; Q6_K 1.2e-7 against 1.7e-7, its hi
 // parts in two sums of 8 steps).
 //
 // Q6_K: u = sc (q - 32) has up to 13 bits, so its fp16 rounding v = fp16(u) is
@@ -99,7 +99,6 @@ __device__ __forceinline__ void min_ratio(float &d, float dm, float &ratio) {
 template <> struct SxtW<Q4_K> {
   static constexpr uint32_t NI = 5, UNITS = 1, BB = 144;
   static constexpr bool REM = false;
-  static constexpr int FB = 2;          // tiles of 32 rows per wave
   static constexpr bool SEP = false;
   uint32_t q[16], sc[2], mi[2];
   float d, ratio;
@@ -141,7 +140,6 @@ template <> struct SxtW<Q4_K> {
 template <> struct SxtW<Q2_K> {
   static constexpr uint32_t NI = 3, UNITS = 1, BB = 84;
   static constexpr bool REM = false;
-  static constexpr int FB = 2;          // tiles of 32 rows per wave
   static constexpr bool SEP = false;
   uint32_t q[8], sc[4];
   float d, ratio;
@@ -188,7 +186,6 @@ template <> struct SxtW<Q2_K> {
 template <> struct SxtW<IQ2_XXS> {
   static constexpr uint32_t NI = 3, UNITS = 1, BB = 66;
   static constexpr bool REM = false;
-  static constexpr int FB = 1;          // tiles of 32 rows per wave
   static constexpr bool SEP = true;
   uint32_t g[8], sc;   // g[i]: steps 2 i and 2 i + 1, 16 bits each: index | field << 8
   float d, ratio;
@@ -243,7 +240,6 @@ template <> struct SxtW<IQ2_XXS> {
 template <> struct SxtW<Q6_K> {
   static constexpr uint32_t NI = 5, UNITS = 2, BB = 210;
   static constexpr bool REM = true;
-  static constexpr int FB = 1;          // tiles of 32 rows per wave
   static constexpr bool SEP = true;
   uint32_t ql[8], qh[4], sc[2];
   float d, ratio;
@@ -307,18 +303,13 @@ __device__ __forceinline__ void wait_vm_lds() {
 
 constexpr uint32_t kTokTile = 64;    // tokens per workgroup: 4 tiles of 16 of the prepared x
 
-template <int TYPE>
-constexpr uint32_t sxt_rows() {      // rows per workgroup: 4 groups of 32 FB
-  static_assert(sxt_row_tile(TYPE) == 128u * SxtW<TYPE>::FB, "row tile");
-  return sxt_row_tile(TYPE);
-}
-
-template <int TYPE>
+// FB: tiles of 32 rows per wave, a workgroup having 4 groups of 32 FB rows.
+template <int TYPE, int FB>
 struct SxtLds {
   static constexpr uint32_t XG = 2u * 4u * 4096u;                   // 4 steps of 64 tokens, for each k slice
   static constexpr uint32_t WR = SxtW<TYPE>::NI * 1024u;            // raw weights of 32 rows
   static constexpr uint32_t TAB = TYPE == IQ2_XXS ? 2048u : 0u;
-  static constexpr uint32_t X0 = TAB, W0 = X0 + 2u * XG, M0 = W0 + 8u * SxtW<TYPE>::FB * WR;
+  static constexpr uint32_t X0 = TAB, W0 = X0 + 2u * XG, M0 = W0 + 8u * FB * WR;
   static constexpr uint32_t P0 = M0 + (sx_mins<TYPE>() ? 8192u : 0u);   // group sums of a block, for each k slice
   static constexpr uint32_t LOOP = P0 + 1024u;                      // block scales: 2 blocks x 2 slices x 64 tokens
   static constexpr uint32_t RED = 8u * 8192u + 16u;                 // the waves' sums handed over
@@ -330,17 +321,17 @@ __device__ __forceinline__ float16v mma(half8 a, half8 b, float16v c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }
 
-template <int TYPE>
+template <int TYPE, int FB>
 __global__ __launch_bounds__(512) void k_sxt(WeightView wv, const uint8_t *__restrict__ xa,
                                              const float *__restrict__ xp, float *__restrict__ y, uint32_t tokens,
                                              uint32_t xa_bytes, uint32_t xp_bytes, uint32_t row_tiles,
                                              uint32_t tok_tiles, uint32_t ksl, float *__restrict__ part,
                                              uint32_t *__restrict__ cnt) {
   using W = SxtW<TYPE>;
-  using L = SxtLds<TYPE>;
+  using L = SxtLds<TYPE, FB>;
   constexpr bool MINS = sx_mins<TYPE>();
   constexpr uint32_t NS = sx_slots<TYPE>();
-  constexpr int FB = W::FB;
+  static_assert(FB == 1 || (FB == 2 && !W::SEP), "registers");
   constexpr uint32_t SU = 16u / W::UNITS;        // steps of a unit
   constexpr uint32_t WI = FB * W::NI;            // a wave's loads of a unit's weights
   constexpr uint32_t XI = 4u;                    // and of a group's x
@@ -354,7 +345,7 @@ __global__ __launch_bounds__(512) void k_sxt(WeightView wv, const uint8_t *__res
   uint32_t u = blockIdx.x;
   if (nwg % 8u == 0u) u = (blockIdx.x % 8u) * (nwg / 8u) + blockIdx.x / 8u;
   const uint32_t z = u / ntiles, lin = u - z * ntiles;
-  const uint32_t tt0 = lin % tok_tiles, r0 = (lin / tok_tiles) * sxt_rows<TYPE>() + 32u * FB * rg;
+  const uint32_t tt0 = lin % tok_tiles, r0 = (lin / tok_tiles) * (128u * FB) + 32u * FB * rg;
   const uint32_t rows = wv.rows, nb = wv.k / 256u;
   const uint32_t bl = z * nb / ksl, bh = (z + 1u) * nb / ksl, iters = (bh - bl + 1u) / 2u;
 
@@ -599,7 +590,7 @@ __global__ __launch_bounds__(512) void k_sxt(WeightView wv, const uint8_t *__res
     // k slices over workgroups, as in eff_gemm_sx.hip: the last of the tile's
     // ksl workgroups to arrive adds the slices in slice order
     constexpr int kSc1 = 16;   // cache policy bit 4: sc1
-    constexpr uint32_t NE = kTokTile * sxt_rows<TYPE>();
+    constexpr uint32_t NE = kTokTile * 128u * FB;
     uint32_t *const arrived = (uint32_t *)(lds + L::BYTES - 16u);
     const rsrc_t prs = make_rsrc(part + (uint64_t)lin * ksl * NE, (uint64_t)ksl * NE * 4u);
     auto off = [&](uint32_t zz, uint32_t a, uint32_t v4) {
@@ -646,12 +637,12 @@ struct SxtPlan {
   uint32_t row_tiles, tok_tiles, ksl;
 };
 
-SxtPlan sxt_plan(const WeightView &wv, uint32_t tokens, uint32_t ksl) {
-  return {(wv.rows + sxt_row_tile(wv.type) - 1u) / sxt_row_tile(wv.type), (tokens + kTokTile - 1u) / kTokTile,
+SxtPlan sxt_plan(const WeightView &wv, uint32_t tokens, uint32_t fb, uint32_t ksl) {
+  return {(wv.rows + 128u * fb - 1u) / (128u * fb), (tokens + kTokTile - 1u) / kTokTile,
           (uint32_t)max(1u, min(ksl, wv.k / 256u))};
 }
 
-template <int TYPE>
+template <int TYPE, int FB>
 hipError_t sxt_go(const WeightView &wv, const uint8_t *xa, const float *xp, uint32_t tiles, float *y,
                   uint32_t tokens, const SxtPlan &p, void *sk, hipStream_t s) {
   const uint64_t nb = wv.k / 256u, xb = (uint64_t)tiles * nb * sx_slots<TYPE>() * 1024u;
@@ -659,29 +650,36 @@ hipError_t sxt_go(const WeightView &wv, const uint8_t *xa, const float *xp, uint
   if (p.ksl > 1u && (!sk || (uint64_t)p.row_tiles * p.tok_tiles > kSliceCntBytes / 4u)) return hipErrorInvalidValue;
   uint32_t *cnt = (uint32_t *)sk;
   float *part = sk ? (float *)((uint8_t *)sk + kSliceCntBytes) : nullptr;
-  hipLaunchKernelGGL((k_sxt<TYPE>), dim3(p.row_tiles * p.tok_tiles * p.ksl), dim3(512), 0, s, wv, xa, xp, y,
+  hipLaunchKernelGGL((k_sxt<TYPE, FB>), dim3(p.row_tiles * p.tok_tiles * p.ksl), dim3(512), 0, s, wv, xa, xp, y,
                      tokens, (uint32_t)xb, (uint32_t)(tiles * nb * 64u), p.row_tiles, p.tok_tiles, p.ksl, part, cnt);
   return hipGetLastError();
 }
 
 }  // namespace
 
-size_t sxt_sk_bytes(const WeightView &wv, uint32_t tokens, uint32_t ksl) {
-  const SxtPlan p = sxt_plan(wv, tokens, ksl);
+size_t sxt_sk_bytes(const WeightView &wv, uint32_t tokens, uint32_t fb, uint32_t ksl) {
+  const SxtPlan p = sxt_plan(wv, tokens, fb, ksl);
   if (p.ksl < 2u) return 0;
-  return kSliceCntBytes + (size_t)p.row_tiles * p.tok_tiles * p.ksl * (kTokTile * sxt_row_tile(wv.type) * 4u);
+  return kSliceCntBytes + (size_t)p.row_tiles * p.tok_tiles * p.ksl * (kTokTile * 128u * fb * 4u);
 }
 
 hipError_t launch_sxt(const WeightView &wv, const void *xa, const void *xp, uint32_t tiles, float *y,
-                      uint32_t tokens, uint32_t ksl, void *sk, hipStream_t s) {
-  const SxtPlan p = sxt_plan(wv, tokens, ksl);
+                      uint32_t tokens, uint32_t fb, uint32_t ksl, void *sk, hipStream_t s) {
+  const SxtPlan p = sxt_plan(wv, tokens, fb, ksl);
   const uint8_t *a = (const uint8_t *)xa;
   const float *b = (const float *)xp;
+  if (fb == 2u) {
+    switch (wv.type) {
+      case Q4_K: return sxt_go<Q4_K, 2>(wv, a, b, tiles, y, tokens, p, sk, s);
+      case Q2_K: return sxt_go<Q2_K, 2>(wv, a, b, tiles, y, tokens, p, sk, s);
+      default: return hipErrorInvalidValue;
+    }
+  }
   switch (wv.type) {
-    case Q4_K: return sxt_go<Q4_K>(wv, a, b, tiles, y, tokens, p, sk, s);
-    case Q6_K: return sxt_go<Q6_K>(wv, a, b, tiles, y, tokens, p, sk, s);
-    case Q2_K: return sxt_go<Q2_K>(wv, a, b, tiles, y, tokens, p, sk, s);
-    case IQ2_XXS: return sxt_go<IQ2_XXS>(wv, a, b, tiles, y, tokens, p, sk, s);
+    case Q4_K: return sxt_go<Q4_K, 1>(wv, a, b, tiles, y, tokens, p, sk, s);
+    case Q6_K: return sxt_go<Q6_K, 1>(wv, a, b, tiles, y, tokens, p, sk, s);
+    case Q2_K: return sxt_go<Q2_K, 1>(wv, a, b, tiles, y, tokens, p, sk, s);
+    case IQ2_XXS: return sxt_go<IQ2_XXS, 1>(wv, a, b, tiles, y, tokens, p, sk, s);
     default: return hipErrorInvalidValue;
   }
 }

@@ -150,13 +150,12 @@ hipError_t launch_sx_prepared(const WeightView &wv, const void *xprep, float *y,
                               uint32_t ksl_opt, void *sk, hipStream_t stream);
 
 // The split-x product over LDS-shared tiles (eff_gemm_sxt.hip; Q2_K, Q4_K,
-// IQ2_XXS, Q6_K): 64 tokens x sxt_row_tile rows per workgroup, k in ksl slices
-// over workgroups; x prepared for `tiles` token tiles of 16 (a multiple of 4, xp
-// the tokens' block scales).
-constexpr uint32_t sxt_row_tile(int type) { return type == Q6_K || type == IQ2_XXS ? 128u : 256u; }
-size_t sxt_sk_bytes(const WeightView &wv, uint32_t tokens, uint32_t ksl);
+// IQ2_XXS, Q6_K): 64 tokens x 128 fb rows per workgroup (fb 1; 2 also for Q2_K
+// and Q4_K), k in ksl slices over workgroups; x prepared for `tiles` token tiles
+// of 16 (a multiple of 4, xp the tokens' block scales).
+size_t sxt_sk_bytes(const WeightView &wv, uint32_t tokens, uint32_t fb, uint32_t ksl);
 hipError_t launch_sxt(const WeightView &wv, const void *xa, const void *xp, uint32_t tiles, float *y,
-                      uint32_t tokens, uint32_t ksl, void *sk, hipStream_t stream);
+                      uint32_t tokens, uint32_t fb, uint32_t ksl, void *sk, hipStream_t stream);
 
 // The reference CPU path's arithmetic for Q8_0 (eff_cpu_path.hip): x into
 // 40-byte 8-bit blocks in `act` (cpu_path_act_bytes(...)), then per row and
