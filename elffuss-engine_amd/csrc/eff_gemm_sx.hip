@@ -524,7 +524,10 @@ __global__ __launch_bounds__(NW * 64) void k_sx(WeightView wv, const uint8_t *__
   // offsets per lane: 3 steps ahead at 4 token tiles keep it within the VGPRs;
   // the types folded per group of steps hold more state: fewer steps ahead)
   constexpr bool MS = W::FG < 16;
-  constexpr uint32_t P = TT == 1 ? 16u : TT == 2 ? (MS ? 4u : 8u) : TT == 3 ? (RF == 1 ? 4u : 5u) : TYPE == Q4_K ? 3u : MS ? 2u : 4u;
+  constexpr uint32_t P = TT == 1   ? 16u
+                         : TT == 2 ? (MS ? 4u : 8u)
+                         : TT == 3 ? (RF == 1 ? 4u : 5u)
+                                   : (TYPE == Q4_K ? 3u : MS ? 2u : 4u);
   constexpr uint32_t ROWS = L::ROWS, ND = L::ND;
   __shared__ __align__(16) uint8_t lds_s[FX ? 16u : L::BYTES];
   extern __shared__ __align__(16) uint8_t lds_d[];
@@ -869,9 +872,11 @@ uint32_t sxt_choose(const WeightView &wv, uint32_t tokens, double rounds, uint32
                         // sums of all slices, per 1e6 values of x (launch 0: not built)
   };
   static const Fit fits[] = {
-      {Q4_K, {4.30, 1.84, 0.209, 2.28, 3.42}, {{1.48, 6.22, 3.76, 2.20, 1.61, 3.78}, {0.17, 9.37, 6.90, 4.14, 1.84, 2.88}}},
+      {Q4_K, {4.30, 1.84, 0.209, 2.28, 3.42},
+       {{1.48, 6.22, 3.76, 2.20, 1.61, 3.78}, {0.17, 9.37, 6.90, 4.14, 1.84, 2.88}}},
       {Q6_K, {4.30, 2.45, 0.356, 2.03, 3.07}, {{1.72, 5.62, 5.09, 1.80, 1.92, 3.29}, {0}}},
-      {Q2_K, {4.22, 1.57, 0.193, 2.16, 3.76}, {{2.15, 5.09, 3.57, 1.75, 1.62, 3.73}, {1.32, 7.92, 6.20, 2.70, 1.87, 3.07}}},
+      {Q2_K, {4.22, 1.57, 0.193, 2.16, 3.76},
+       {{2.15, 5.09, 3.57, 1.75, 1.62, 3.73}, {1.32, 7.92, 6.20, 2.70, 1.87, 3.07}}},
       {IQ2_XXS, {4.78, 1.35, 0.189, 2.12, 3.68}, {{2.36, 5.06, 4.20, 1.76, 1.63, 3.26}, {0}}}};
   if (tokens <= 32u) return 0u;   // the x scratch then holds less than the kernel's 64 tokens
   const uint64_t nb = wv.k / 256u, xb = (uint64_t)sx_tile_count(wv.type, tokens) * nb * 17u * 1024u;
@@ -1037,7 +1042,7 @@ hipError_t sx_type(const WeightView &wv, const float *x, float *y, uint32_t toke
     if (sx_fx(TYPE, tokens, cfg, p, wv.k)) return sx_go_fx<TYPE>(wv, x, y, tokens, p, nullptr, s);
   if constexpr (TYPE == Q8_0 || TYPE == Q8_0R || TYPE == Q6_K)
     if (sx_fx_plain(TYPE, tokens, cfg, p, wv.k)) return sx_go_fx<TYPE>(wv, x, y, tokens, p, sk, s);
-  const uint32_t tiles = sx_tile_count(TYPE, tokens), nb = wv.k / 256u;   // blocks of 256 weights
+  const uint32_t tiles = p.shared ? sx_tile_count(TYPE, tokens) : p.groups * p.tt, nb = wv.k / 256u;
   uint8_t *xa = scratch;
   float *xp = (float *)(scratch + (uint64_t)tiles * nb * sx_slots<TYPE>() * 1024u);
   hipLaunchKernelGGL((k_sx_prep<TYPE>), dim3(nb, tiles * 4u), dim3(256), 0, s, x, tokens, wv.k, xa, xp);

@@ -18,7 +18,8 @@ REL = 2.0 ** -20
 # (type, rows, k, tokens): shapes at which the planner takes the shared tiles, of
 # one and (Q4_K, Q2_K) two row tiles per wave, whole and in 2 to 8 k slices
 SHAPES = [("Q4_K", 513, 256, 4000), ("Q4_K", 1000, 4352, 1000), ("Q4_K", 513, 8192, 501), ("Q4_K", 777, 768, 4000),
-          ("Q4_K", 3000, 2304, 449), ("Q4_K", 700, 4352, 1500), ("Q2_K", 513, 256, 4000), ("Q2_K", 513, 8192, 501), ("Q2_K", 3000, 768, 1000),
+          ("Q4_K", 3000, 2304, 449), ("Q4_K", 700, 4352, 1500), ("Q2_K", 513, 256, 4000),
+          ("Q2_K", 513, 8192, 501), ("Q2_K", 3000, 768, 1000),
           ("Q6_K", 1000, 256, 520), ("Q6_K", 777, 768, 1000), ("Q6_K", 513, 2304, 1000), ("Q6_K", 1000, 8192, 65),
           ("IQ2_XXS", 777, 256, 2000), ("IQ2_XXS", 513, 4352, 501)]
 
