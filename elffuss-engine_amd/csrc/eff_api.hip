@@ -80,6 +80,8 @@ struct eff_ctx {
   int64_t sx_split = 0;             // split-x k slices (0: automatic)
   void *sk_scratch = nullptr;       // k-slice counters and sums (GEMM and split-x)
   size_t sk_scratch_bytes = 0;
+  void *sxt_scratch = nullptr;      // the same of the LDS-shared split-x tiles (sx_slices)
+  size_t sxt_scratch_bytes = 0;
   hipEvent_t order_ev = nullptr;    // orders a newly set stream after the previous one
   int64_t sx_min_tokens = 0;        // 0: the measured default (sx_routes)
   void *act_scratch = nullptr;      // x in the CPU path's 8-bit blocks (eff_qmatmul_cpu_path)
@@ -339,18 +341,51 @@ int sk_scratch(eff_ctx *ctx, const WeightView &wv, uint32_t tokens, uint32_t pla
                                    (uint32_t)ctx->gemm_split), out);
 }
 
+// The k-slice scratch of a split-x product and the configuration it runs in.
+// The slices of the LDS-shared tiles have a buffer of their own, allocated once
+// at the largest automatic size (42 MB), so that no later call frees what an
+// earlier recording reads. Where it cannot be had (the stream is recorded and
+// no call before needed it, or no memory) the call takes k_sx, as calls of
+// these shapes do without slices.
+int sx_slices(eff_ctx *ctx, const WeightView &wv, uint32_t tokens, int *cfg, void **sk) {
+  const uint32_t ks = (uint32_t)ctx->sx_split;
+  *cfg = (int)ctx->sx_config;
+  *sk = nullptr;
+  if (sx_shared(wv, tokens, *cfg, ks)) {
+    const size_t need = sx_sk_bytes(wv, tokens, *cfg, ks);
+    if (!need) return EFF_OK;
+    if (need > ctx->sxt_scratch_bytes) {
+      hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+      EFF_HIP(ctx, hipStreamIsCapturing(ctx->stream, &cs));
+      const size_t size = need > kSxtSkBytes ? need : kSxtSkBytes;
+      if (cs == hipStreamCaptureStatusNone) {
+        if (grow(ctx, &ctx->sxt_scratch, &ctx->sxt_scratch_bytes, size, "k-slice") == EFF_OK)
+          EFF_HIP(ctx, hipMemsetAsync(ctx->sxt_scratch, 0, kSliceCntBytes, ctx->stream));
+        else
+          (void)hipGetLastError();
+      }
+    }
+    if (need <= ctx->sxt_scratch_bytes) {
+      *sk = ctx->sxt_scratch;
+      return EFF_OK;
+    }
+    *cfg = kSxUnshared;
+  }
+  return sk_get(ctx, sx_sk_bytes(wv, tokens, *cfg, ks), sk);
+}
+
 // Split-x matrix-core product (Q2_K, Q4_K, IQ2_XXS, Q8_0, Q8_0R, Q6_K from 2
 // tokens, f32-accurate).
 int run_sx(eff_ctx *ctx, const WeightView &wv, const float *x, float *y, uint32_t tokens) {
   int rc = grow(ctx, &ctx->sx_scratch, &ctx->sx_scratch_bytes, sx_x_bytes(wv.type, tokens, wv.k), "split-x");
   if (rc) return rc;
-  const uint32_t ks = (uint32_t)ctx->sx_split;
   void *sk;
-  if ((rc = sk_get(ctx, sx_sk_bytes(wv, tokens, (int)ctx->sx_config, ks), &sk))) return rc;
-  hipError_t e = launch_sx(wv, x, y, tokens, ctx->sx_scratch, (int)ctx->sx_config, ks, sk, ctx->stream);
+  int cfg;
+  if ((rc = sx_slices(ctx, wv, tokens, &cfg, &sk))) return rc;
+  hipError_t e = launch_sx(wv, x, y, tokens, ctx->sx_scratch, cfg, (uint32_t)ctx->sx_split, sk, ctx->stream);
   if (e != hipSuccess) return hip_fail(ctx, e, "split-x launch");
   ++ctx->stats.split;
-  if (sx_x_layout(wv, tokens, (int)ctx->sx_config, ks)) ++ctx->stats.split_x;
+  if (sx_x_layout(wv, tokens, (int)ctx->sx_config, (uint32_t)ctx->sx_split)) ++ctx->stats.split_x;
   return EFF_OK;
 }
 
@@ -517,6 +552,7 @@ int eff_shutdown(eff_ctx *ctx) {
   if (ctx->sx_scratch) (void)hipFree(ctx->sx_scratch);
   if (ctx->act_scratch) (void)hipFree(ctx->act_scratch);
   if (ctx->sk_scratch) (void)hipFree(ctx->sk_scratch);
+  if (ctx->sxt_scratch) (void)hipFree(ctx->sxt_scratch);
   if (ctx->order_ev) (void)hipEventDestroy(ctx->order_ev);
   for (auto &p : ctx->stage_pend) (void)hipEventDestroy(p.ev);
   for (hipEvent_t ev : ctx->events) (void)hipEventDestroy(ev);
@@ -1113,9 +1149,9 @@ int eff_qmatmul_prepared(eff_ctx *ctx, int type, eff_buf *w, eff_buf *xp, eff_bu
   hipError_t e;
   if (l & kSxLayout) {
     void *sk;
-    if ((rc = sk_get(ctx, sx_sk_bytes(wv, tokens, (int)ctx->sx_config, (uint32_t)ctx->sx_split), &sk))) return rc;
-    e = launch_sx_prepared(wv, xp->ptr, (float *)y->ptr, tokens, (int)ctx->sx_config, (uint32_t)ctx->sx_split, sk,
-                           ctx->stream);
+    int cfg;
+    if ((rc = sx_slices(ctx, wv, tokens, &cfg, &sk))) return rc;
+    e = launch_sx_prepared(wv, xp->ptr, (float *)y->ptr, tokens, cfg, (uint32_t)ctx->sx_split, sk, ctx->stream);
     ++ctx->stats.split;
   } else {
     void *sk;

@@ -891,7 +891,7 @@ uint32_t sxt_choose(const WeightView &wv, uint32_t tokens, double rounds, uint32
       if (c[0] == 0.0) continue;
       const uint64_t tiles = (uint64_t)((wv.rows + 128u * i - 1u) / (128u * i)) * ((tokens + 63u) / 64u);
       for (uint32_t s : {1u, 2u, 3u, 4u, 6u, 8u}) {
-        if (s > 1u && (tiles * s > 640u || nb / s < 2u)) break;
+        if (s > 1u && (tiles * s > kSxtSliceWgs || nb / s < 2u)) break;
         const uint64_t r = (tiles * s + 255u) / 256u, pairs = ((nb + s - 1u) / s + 1u) / 2u;
         const double t = c[0] + (double)r * (c[1] + c[2] * (double)pairs) + (s > 1u ? c[3] + c[4] * out * s : 0.0) +
                          c[5] * xk;
@@ -904,6 +904,8 @@ uint32_t sxt_choose(const WeightView &wv, uint32_t tokens, double rounds, uint32
 }
 
 SxPlan sx_plan(const WeightView &wv, uint32_t tokens, int cfg, uint32_t ksl_opt) {
+  const bool share = cfg == 0;
+  if (cfg == kSxUnshared) cfg = 0;
   SxPlan p;
   sx_tiles(wv.type, tokens, p.tt, p.groups);
   // 32 rows x 8 waves, or 64 x 4 (the types of up to 4 token tiles, from 9
@@ -949,7 +951,7 @@ SxPlan sx_plan(const WeightView &wv, uint32_t tokens, int cfg, uint32_t ksl_opt)
   // the LDS-shared tiles, where they are estimated to be the faster
   const double rounds = p.ksl > 1u ? (p.cfg ? 1.75 : 1.0) * ((wgs * p.ksl + 255u) / 256u) : p.cfg ? t64 : t32;
   uint32_t shared_ksl = 1u;
-  p.shared = cfg == 0 ? sxt_choose(wv, tokens, rounds, (nb + p.ksl - 1u) / p.ksl * p.tt, p.ksl > 1u, shared_ksl) : 0u;
+  p.shared = share ? sxt_choose(wv, tokens, rounds, (nb + p.ksl - 1u) / p.ksl * p.tt, p.ksl > 1u, shared_ksl) : 0u;
   if (p.shared) p.ksl = max(1u, min(ksl_opt ? ksl_opt : shared_ksl, nb));
   return p;
 }
@@ -1075,6 +1077,10 @@ size_t sx_sk_bytes(const WeightView &wv, uint32_t tokens, int cfg, uint32_t ksl_
   if (p.ksl < 2u || sx_fx(wv.type, tokens, cfg, p, wv.k)) return 0;
   const uint64_t ne = (uint64_t)p.tt * (p.cfg ? 2u : 1u) * 512u;   // sums per workgroup
   return kSliceCntBytes + (size_t)((uint64_t)p.row_tiles * p.groups * p.ksl * ne * 4u);
+}
+
+bool sx_shared(const WeightView &wv, uint32_t tokens, int cfg, uint32_t ksl_opt) {
+  return sx_plan(wv, tokens, cfg, ksl_opt).shared != 0u;
 }
 
 uint32_t sx_x_layout(const WeightView &wv, uint32_t tokens, int cfg, uint32_t ksl_opt) {
