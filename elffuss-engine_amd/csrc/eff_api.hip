@@ -343,10 +343,10 @@ int sk_scratch(eff_ctx *ctx, const WeightView &wv, uint32_t tokens, uint32_t pla
 
 // The k-slice scratch of a split-x product and the configuration it runs in.
 // The slices of the LDS-shared tiles have a buffer of their own, allocated once
-// at the largest automatic size (42 MB), so that no later call frees what an
-// earlier recording reads. Where it cannot be had (the stream is recorded and
-// no call before needed it, or no memory) the call takes k_sx, as calls of
-// these shapes do without slices.
+// at the largest size a plan of theirs has (42 MB) and never replaced, so that no
+// later call frees what an earlier recording reads. Where it cannot be had (the
+// stream is recorded and no call before needed it, or no memory) the call takes
+// k_sx.
 int sx_slices(eff_ctx *ctx, const WeightView &wv, uint32_t tokens, int *cfg, void **sk) {
   const uint32_t ks = (uint32_t)ctx->sx_split;
   *cfg = (int)ctx->sx_config;
@@ -357,9 +357,8 @@ int sx_slices(eff_ctx *ctx, const WeightView &wv, uint32_t tokens, int *cfg, voi
     if (need > ctx->sxt_scratch_bytes) {
       hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
       EFF_HIP(ctx, hipStreamIsCapturing(ctx->stream, &cs));
-      const size_t size = need > kSxtSkBytes ? need : kSxtSkBytes;
       if (cs == hipStreamCaptureStatusNone) {
-        if (grow(ctx, &ctx->sxt_scratch, &ctx->sxt_scratch_bytes, size, "k-slice") == EFF_OK)
+        if (grow(ctx, &ctx->sxt_scratch, &ctx->sxt_scratch_bytes, kSxtSkBytes, "k-slice") == EFF_OK)
           EFF_HIP(ctx, hipMemsetAsync(ctx->sxt_scratch, 0, kSliceCntBytes, ctx->stream));
         else
           (void)hipGetLastError();
@@ -1122,6 +1121,17 @@ int eff_qmatmul_prepare_x(eff_ctx *ctx, int type, eff_buf *x, eff_buf *xp, uint3
     ++ctx->stats.gemm_x;
   }
   if (e != hipSuccess) return hip_fail(ctx, e, "matmul prepare x launch");
+  return EFF_OK;
+}
+
+int eff_split_plan(int type, uint32_t rows, uint32_t k, uint32_t tokens, int config, uint32_t slices,
+                   eff_split_plan_info *out) {
+  WeightView wv;
+  if (!out || config < 0 || config > 3) return EFF_E_INVALID;
+  const int rc = matmul_prepared_view(nullptr, type, rows, k, tokens, wv, "split plan");
+  if (rc) return rc;
+  if (!sx_applies(wv, tokens)) return EFF_NOT_APPLICABLE;
+  sx_describe(wv, tokens, config, slices, out);
   return EFF_OK;
 }
 

@@ -952,7 +952,12 @@ SxPlan sx_plan(const WeightView &wv, uint32_t tokens, int cfg, uint32_t ksl_opt)
   const double rounds = p.ksl > 1u ? (p.cfg ? 1.75 : 1.0) * ((wgs * p.ksl + 255u) / 256u) : p.cfg ? t64 : t32;
   uint32_t shared_ksl = 1u;
   p.shared = share ? sxt_choose(wv, tokens, rounds, (nb + p.ksl - 1u) / p.ksl * p.tt, p.ksl > 1u, shared_ksl) : 0u;
-  if (p.shared) p.ksl = max(1u, min(ksl_opt ? ksl_opt : shared_ksl, nb));
+  if (p.shared) {
+    // a forced count whose sums the slices' buffer cannot hold stays on k_sx
+    const uint32_t ksl = max(1u, min(ksl_opt ? ksl_opt : shared_ksl, nb));
+    if (sxt_sk_bytes(wv, tokens, p.shared, ksl) <= kSxtSkBytes) p.ksl = ksl;
+    else p.shared = 0u;
+  }
   return p;
 }
 
@@ -1081,6 +1086,15 @@ size_t sx_sk_bytes(const WeightView &wv, uint32_t tokens, int cfg, uint32_t ksl_
 
 bool sx_shared(const WeightView &wv, uint32_t tokens, int cfg, uint32_t ksl_opt) {
   return sx_plan(wv, tokens, cfg, ksl_opt).shared != 0u;
+}
+
+void sx_describe(const WeightView &wv, uint32_t tokens, int cfg, uint32_t ksl_opt, eff_split_plan_info *out) {
+  const SxPlan p = sx_plan(wv, tokens, cfg, ksl_opt);
+  out->shared = p.shared ? 1u : 0u;
+  out->rows = p.shared ? 128u * p.shared : p.cfg ? 64u : 32u;
+  out->slices = p.ksl;
+  out->prepares_x = !sx_fx(wv.type, tokens, cfg, p, wv.k) && !sx_fx_plain(wv.type, tokens, cfg, p, wv.k);
+  out->slice_bytes = sx_sk_bytes(wv, tokens, cfg, ksl_opt);
 }
 
 uint32_t sx_x_layout(const WeightView &wv, uint32_t tokens, int cfg, uint32_t ksl_opt) {

@@ -7,6 +7,7 @@
 
 #include <atomic>
 
+#include "../../include/elffuss_amd.h"
 #include "eff_formats.h"
 
 namespace eff {
@@ -136,6 +137,7 @@ size_t sx_sk_bytes(const WeightView &wv, uint32_t tokens, int cfg, uint32_t ksl_
 // Whether the call takes the LDS-shared tiles (k_sxt); with cfg kSxUnshared none does.
 constexpr int kSxUnshared = -1;
 bool sx_shared(const WeightView &wv, uint32_t tokens, int cfg, uint32_t ksl_opt);
+void sx_describe(const WeightView &wv, uint32_t tokens, int cfg, uint32_t ksl_opt, eff_split_plan_info *out);
 hipError_t launch_sx(const WeightView &wv, const float *x, float *y, uint32_t tokens, void *scratch, int cfg,
                      uint32_t ksl_opt, void *sk, hipStream_t stream);
 // The same product in two halves, so that one preparation of x serves every
@@ -158,7 +160,8 @@ hipError_t launch_sx_prepared(const WeightView &wv, const void *xprep, float *y,
 // of 16 (a multiple of 4, xp the tokens' block scales).
 size_t sxt_sk_bytes(const WeightView &wv, uint32_t tokens, uint32_t fb, uint32_t ksl);
 // Automatic k slices keep within 640 workgroups; the scratch they then take at
-// most (64 tokens x 256 rows of sums each).
+// most (64 tokens x 256 rows of sums each), and what a context holds for them: a
+// forced count that would need more takes k_sx.
 constexpr uint32_t kSxtSliceWgs = 640u;
 constexpr size_t kSxtSkBytes = kSliceCntBytes + (size_t)kSxtSliceWgs * 64u * 256u * 4u;
 hipError_t launch_sxt(const WeightView &wv, const void *xa, const void *xp, uint32_t tiles, float *y,

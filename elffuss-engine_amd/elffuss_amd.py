@@ -47,6 +47,11 @@ class Stats(ctypes.Structure):
                 ("gemm_x", ctypes.c_uint64), ("split_x", ctypes.c_uint64), ("cpu_path", ctypes.c_uint64)]
 
 
+class SplitPlan(ctypes.Structure):
+    _fields_ = [("shared", ctypes.c_uint32), ("rows", ctypes.c_uint32), ("slices", ctypes.c_uint32),
+                ("prepares_x", ctypes.c_uint32), ("slice_bytes", ctypes.c_uint64)]
+
+
 _lib = None
 
 
@@ -112,6 +117,7 @@ def lib():
         "eff_qmatmul_cpu_path": ([p, i32, p, p, p, u32, u32, u32], i32),
         "eff_qmatmul_x_layout": ([p, i32, u32, u32, u32, ctypes.POINTER(sz), ctypes.POINTER(u32)], i32),
         "eff_qmatmul_prepare_x": ([p, i32, p, p, u32, u32, u32], i32),
+        "eff_split_plan": ([i32, u32, u32, u32, i32, u32, ctypes.POINTER(SplitPlan)], i32),
         "eff_qmatmul_prepared": ([p, i32, p, p, p, u32, u32, u32], i32),
         "eff_qgemv_multi": ([p, i32, i32, u32, ctypes.POINTER(p), p, ctypes.POINTER(p), ctypes.POINTER(u32), u32, u32],
                             i32),
@@ -139,7 +145,7 @@ EXPORTED = ("eff_type_from_name eff_type_name eff_type_geometry eff_init eff_shu
             "eff_read_begin eff_read_end eff_read_poll eff_read_error eff_read_release "
             "eff_bytes_reordered eff_bytes_buffer_r eff_blocks_from_buffer eff_scales_from eff_buf_mark_r "
             "eff_buf_blocks_r eff_buf_write_r eff_repack eff_unrepack eff_quantize eff_fill_normal eff_qmatmul eff_qgemv "
-            "eff_qgemm eff_qgemm_planned eff_gemm_x_layout eff_gemm_prepare_x eff_qgemm_prepared eff_qmatmul_x_layout eff_qmatmul_prepare_x eff_qmatmul_prepared eff_qmatmul_cpu_path eff_qgemv_multi eff_dequant eff_gather eff_gather_norm eff_topk eff_topk_noalloc eff_qgemv_topk eff_topk_out_bytes eff_read_floor").split()
+            "eff_qgemm eff_qgemm_planned eff_gemm_x_layout eff_gemm_prepare_x eff_qgemm_prepared eff_qmatmul_x_layout eff_qmatmul_prepare_x eff_qmatmul_prepared eff_split_plan eff_qmatmul_cpu_path eff_qgemv_multi eff_dequant eff_gather eff_gather_norm eff_topk eff_topk_noalloc eff_qgemv_topk eff_topk_out_bytes eff_read_floor").split()
 
 
 def type_code(t):
@@ -148,6 +154,17 @@ def type_code(t):
             raise EffError(E_TYPE, f"unsupported quantization type «{t}»")
         return TYPES[t]
     return int(t)
+
+
+def split_plan(t, rows, k, tokens, config=0, slices=0):
+    """What the split-x product runs for a call (no device needed)."""
+    out = SplitPlan()
+    rc = lib().eff_split_plan(type_code(t), rows, k, tokens, config, slices, ctypes.byref(out))
+    if rc == NOT_APPLICABLE:
+        raise NotApplicable()
+    if rc:
+        raise EffError(rc, "split plan")
+    return {f: getattr(out, f) for f, _ in SplitPlan._fields_}
 
 
 def geometry(t):

@@ -317,6 +317,21 @@ int eff_fill_normal(uint32_t seed, float sigma, float *dst, size_t n);
 int eff_qmatmul(eff_ctx *ctx, int type, eff_buf *w, eff_buf *x, eff_buf *y,
                 uint32_t rows, uint32_t k, uint32_t tokens);
 
+/* What the split-x product runs for a call of eff_qmatmul that takes it, under
+ * EFF_OPT_SPLIT_CONFIG = config and EFF_OPT_SPLIT_SLICES = slices (0, 0: the
+ * defaults): a description for tests and tuning, computed on the host without a
+ * device. EFF_NOT_APPLICABLE where the product does not exist (one token, k not a
+ * multiple of 256). No counterpart in the reference. */
+typedef struct eff_split_plan_info {
+  uint32_t shared;       /* 1: LDS-shared tiles of x (prompts), 0: x read by each wave */
+  uint32_t rows;         /* rows per workgroup */
+  uint32_t slices;       /* k slices over workgroups */
+  uint32_t prepares_x;   /* 1: x is prepared by a launch of its own, 0: inside the product */
+  uint64_t slice_bytes;  /* scratch of the slices' counters and sums */
+} eff_split_plan_info;
+int eff_split_plan(int type, uint32_t rows, uint32_t k, uint32_t tokens, int config, uint32_t slices,
+                   eff_split_plan_info *out);
+
 /* eff_qmatmul with x prepared once for several products. The router's
  * split-x product and fp16 GEMM read x in a prepared form (fp16 hi/lo parts
  * with block scales; fp16 tiles); the matmuls of one activation (q, k and v;

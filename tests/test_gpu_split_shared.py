@@ -151,6 +151,42 @@ def test_recorded_without_slice_scratch(eff, orc):
             b.free()
 
 
+def test_forced_slices_leave_a_recording_its_buffer(eff, orc):
+    """A recording of the sliced shared tiles, then eager calls whose forced slice
+    count needs more than the slices' buffer holds (256 tiles x 8): they run the
+    other kernel, and the recording replays its bits."""
+    with eff.Context(0) as ctx:
+        small, big = ("Q6_K", 2048, 8192, 300), ("Q4_K", 8192, 2048, 512)
+        assert eff.split_plan(*small)["shared"] and eff.split_plan(*small)["slices"] > 1
+        assert not eff.split_plan(*big, 0, 8)["shared"]
+        st = []
+        for tname, rows, k, tokens in (small, big):
+            t, data, gguf, n = make_weights(eff, tname, rows, k, 97)
+            x = eff.fill_normal(98, 1.0, tokens * k)
+            st.append((t, ctx.upload(data), ctx.upload(x), ctx.alloc(tokens * rows * 4), product(orc, tname, gguf, n, x, rows, k)))
+        t, wb, xb, yb, ref = st[0]
+        t2, wb2, xb2, yb2, ref2 = st[1]
+        ctx.qmatmul(t2, wb2, xb2, yb2, *big[1:])
+        ctx.qmatmul(t, wb, xb, yb, *small[1:])
+        want = yb.read(np.uint32)
+        assert np.linalg.norm(want.view(np.float32).reshape(ref.shape) - ref) <= REL * np.linalg.norm(ref)
+        ctx.graph_begin()
+        ctx.qmatmul(t, wb, xb, yb, *small[1:])
+        g = ctx.graph_end()
+        ctx.set_option(eff.OPT_SPLIT_SLICES, 8)
+        for _ in range(2):
+            ctx.qmatmul(t2, wb2, xb2, yb2, *big[1:])
+            y2 = yb2.read(np.float32).reshape(ref2.shape)
+            assert np.linalg.norm(y2 - ref2) <= REL * np.linalg.norm(ref2)
+            yb.write(np.zeros(yb.size // 4, np.float32))
+            g.launch()
+            assert np.array_equal(yb.read(np.uint32), want)
+        g.destroy()
+        for _, *bufs, _ in st:
+            for b in bufs:
+                b.free()
+
+
 @pytest.mark.parametrize("tname", ["Q4_K", "Q2_K", "IQ2_XXS"])
 @pytest.mark.parametrize("tokens", [33, 48, 64, 65, 96, 129])
 def test_three_token_tiles(ctx, eff, orc, tname, tokens):
