@@ -80,8 +80,7 @@ struct eff_ctx {
   int64_t sx_split = 0;             // split-x k slices (0: automatic)
   void *sk_scratch = nullptr;       // k-slice counters and sums (GEMM and split-x)
   size_t sk_scratch_bytes = 0;
-  void *sxt_scratch = nullptr;      // the same of the LDS-shared split-x tiles (sx_slices)
-  size_t sxt_scratch_bytes = 0;
+  void *sxt_scratch = nullptr;      // the same of the LDS-shared split-x tiles, kSxtSkBytes (sx_slices)
   hipEvent_t order_ev = nullptr;    // orders a newly set stream after the previous one
   int64_t sx_min_tokens = 0;        // 0: the measured default (sx_routes)
   void *act_scratch = nullptr;      // x in the CPU path's 8-bit blocks (eff_qmatmul_cpu_path)
@@ -342,32 +341,18 @@ int sk_scratch(eff_ctx *ctx, const WeightView &wv, uint32_t tokens, uint32_t pla
 }
 
 // The k-slice scratch of a split-x product and the configuration it runs in.
-// The slices of the LDS-shared tiles have a buffer of their own, allocated once
-// at the largest size a plan of theirs has (42 MB) and never replaced, so that no
-// later call frees what an earlier recording reads. Where it cannot be had (the
-// stream is recorded and no call before needed it, or no memory) the call takes
-// k_sx.
+// The slices of the LDS-shared tiles have a buffer of their own, made with the
+// context at the largest size a plan of theirs has (42 MB): recorded or not,
+// first call or later, a shape runs the same kernel and gives the same bits, and
+// no call frees what a recording reads. A context that found no memory for it
+// takes k_sx for those shapes, always.
 int sx_slices(eff_ctx *ctx, const WeightView &wv, uint32_t tokens, int *cfg, void **sk) {
   const uint32_t ks = (uint32_t)ctx->sx_split;
   *cfg = (int)ctx->sx_config;
   *sk = nullptr;
   if (sx_shared(wv, tokens, *cfg, ks)) {
-    const size_t need = sx_sk_bytes(wv, tokens, *cfg, ks);
-    if (!need) return EFF_OK;
-    if (need > ctx->sxt_scratch_bytes) {
-      hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-      EFF_HIP(ctx, hipStreamIsCapturing(ctx->stream, &cs));
-      if (cs == hipStreamCaptureStatusNone) {
-        if (grow(ctx, &ctx->sxt_scratch, &ctx->sxt_scratch_bytes, kSxtSkBytes, "k-slice") == EFF_OK)
-          EFF_HIP(ctx, hipMemsetAsync(ctx->sxt_scratch, 0, kSliceCntBytes, ctx->stream));
-        else
-          (void)hipGetLastError();
-      }
-    }
-    if (need <= ctx->sxt_scratch_bytes) {
-      *sk = ctx->sxt_scratch;
-      return EFF_OK;
-    }
+    if (!sx_sk_bytes(wv, tokens, *cfg, ks)) return EFF_OK;
+    if ((*sk = ctx->sxt_scratch)) return EFF_OK;
     *cfg = kSxUnshared;
   }
   return sk_get(ctx, sx_sk_bytes(wv, tokens, *cfg, ks), sk);
@@ -527,6 +512,12 @@ int eff_init(int device, eff_ctx **out) {
     return EFF_E_DEVICE;
   }
   ctx->stream = ctx->own;
+  if (hipMalloc(&ctx->sxt_scratch, kSxtSkBytes) != hipSuccess ||
+      hipMemsetAsync(ctx->sxt_scratch, 0, kSliceCntBytes, ctx->own) != hipSuccess) {
+    if (ctx->sxt_scratch) (void)hipFree(ctx->sxt_scratch);
+    ctx->sxt_scratch = nullptr;
+    (void)hipGetLastError();
+  }
   if (device < kMaxDevices) {
     // once per device, with the device current: the address of its copy of
     // the no-alloc scratch (a lookup, not an allocation)

@@ -128,7 +128,9 @@ int eff_type_geometry(int type, uint32_t *block_elems, uint32_t *block_bytes);
 
 /* ---- context -------------------------------------------------------------- */
 
-/* Open a context on HIP device `device` with its own stream (default priority).
+/* Open a context on HIP device `device` with its own stream (default priority) and
+ * 42 MB of device memory for the k slices of the split-x prompts; where that cannot
+ * be had, the context runs those without slices.
  * Replaces requestDevice + createOps (device.js:66-139, ops.js:1604-1633). */
 int eff_init(int device, eff_ctx **out);
 

@@ -98,14 +98,14 @@ def test_shared_tiles_range_and_non_finite(ctx, eff, orc, tname, rows, k, tokens
     wb.free()
 
 
-def test_recorded_without_slice_scratch(eff, orc):
-    """A shape whose shared tiles take k slices, recorded in a context that has no
-    scratch for them yet: the recording takes the unsliced kernel and is not
-    refused; it replays unchanged after eager calls have taken the slices, and so
-    does a recording of the sliced form."""
+def test_recorded_before_any_eager_call_gives_the_eager_bits(eff, orc):
+    """A shape whose shared tiles take k slices, recorded in a context in which no
+    eager call has taken them: the recording runs the same kernel, gives the bits of
+    the eager calls that follow, and replays them unchanged among other products."""
     rows, k, tokens = 2048, 8192, 300
     with eff.Context(0) as ctx:
         t, data, gguf, n = make_weights(eff, "Q6_K", rows, k, 97)
+        assert eff.split_plan(t, rows, k, tokens)["shared"] and eff.split_plan(t, rows, k, tokens)["slices"] > 1
         x = eff.fill_normal(98, 1.0, tokens * k)
         ref = product(orc, "Q6_K", gguf, n, x, rows, k)
         wb, xb, yb = ctx.upload(data), ctx.upload(x), ctx.alloc(tokens * rows * 4)
@@ -113,7 +113,7 @@ def test_recorded_without_slice_scratch(eff, orc):
         xp = ctx.alloc(nb)
         ctx.qmatmul_prepare_x(t, xb, xp, rows, k, tokens)
         ctx.set_option(eff.OPT_SPLIT_CONFIG, 1)
-        ctx.qmatmul(t, wb, xb, yb, rows, k, tokens)      # sizes the x scratch
+        ctx.qmatmul(t, wb, xb, yb, rows, k, tokens)      # sizes the x scratch, by the other kernel
         plain = yb.read(np.uint32)
         ctx.set_option(eff.OPT_SPLIT_CONFIG, 0)
 
@@ -125,27 +125,26 @@ def test_recorded_without_slice_scratch(eff, orc):
                 ctx.qmatmul(t, wb, xb, yb, rows, k, tokens)
             return ctx.graph_end()
 
-        def replays(g, want):
+        graphs = [record(False), record(True)]
+        got = []
+        for g in graphs:
             yb.write(np.zeros(tokens * rows, np.float32))
             g.launch()
-            assert np.array_equal(yb.read(np.uint32), want)
-
-        before = [record(False), record(True)]
-        for g in before:
-            replays(g, plain)
+            got.append(yb.read(np.uint32))
         ctx.qmatmul(t, wb, xb, yb, rows, k, tokens)
-        sliced = yb.read(np.uint32)
-        assert not np.array_equal(sliced, plain)
-        for y in (plain, sliced):
-            assert np.linalg.norm(y.view(np.float32).reshape(tokens, rows) - ref) <= REL * np.linalg.norm(ref)
-        after = [record(False), record(True)]
+        eager = yb.read(np.uint32)
+        assert not np.array_equal(eager, plain)
+        assert np.linalg.norm(eager.view(np.float32).reshape(tokens, rows) - ref) <= REL * np.linalg.norm(ref)
+        for y in got:
+            assert np.array_equal(y, eager)
+        graphs += [record(False), record(True)]
         for _ in range(2):
             ctx.qmatmul(t, wb, xb, yb, rows, k, 129)
-            for g in before:
-                replays(g, plain)
-            for g in after:
-                replays(g, sliced)
-        for g in before + after:
+            for g in graphs:
+                yb.write(np.zeros(tokens * rows, np.float32))
+                g.launch()
+                assert np.array_equal(yb.read(np.uint32), eager)
+        for g in graphs:
             g.destroy()
         for b in (wb, xb, yb, xp):
             b.free()
