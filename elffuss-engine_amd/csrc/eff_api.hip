@@ -369,7 +369,7 @@ int run_sx(eff_ctx *ctx, const WeightView &wv, const float *x, float *y, uint32_
   hipError_t e = launch_sx(wv, x, y, tokens, ctx->sx_scratch, cfg, (uint32_t)ctx->sx_split, sk, ctx->stream);
   if (e != hipSuccess) return hip_fail(ctx, e, "split-x launch");
   ++ctx->stats.split;
-  if (sx_x_layout(wv, tokens, (int)ctx->sx_config, (uint32_t)ctx->sx_split)) ++ctx->stats.split_x;
+  if (sx_prepares_x(wv, tokens, cfg, (uint32_t)ctx->sx_split)) ++ctx->stats.split_x;
   return EFF_OK;
 }
 

@@ -1088,12 +1088,17 @@ bool sx_shared(const WeightView &wv, uint32_t tokens, int cfg, uint32_t ksl_opt)
   return sx_plan(wv, tokens, cfg, ksl_opt).shared != 0u;
 }
 
+bool sx_prepares_x(const WeightView &wv, uint32_t tokens, int cfg, uint32_t ksl_opt) {
+  const SxPlan p = sx_plan(wv, tokens, cfg, ksl_opt);
+  return !sx_fx(wv.type, tokens, cfg, p, wv.k) && !sx_fx_plain(wv.type, tokens, cfg, p, wv.k);
+}
+
 void sx_describe(const WeightView &wv, uint32_t tokens, int cfg, uint32_t ksl_opt, eff_split_plan_info *out) {
   const SxPlan p = sx_plan(wv, tokens, cfg, ksl_opt);
   out->shared = p.shared ? 1u : 0u;
   out->rows = p.shared ? 128u * p.shared : p.cfg ? 64u : 32u;
   out->slices = p.ksl;
-  out->prepares_x = !sx_fx(wv.type, tokens, cfg, p, wv.k) && !sx_fx_plain(wv.type, tokens, cfg, p, wv.k);
+  out->prepares_x = sx_prepares_x(wv, tokens, cfg, ksl_opt);
   out->slice_bytes = sx_sk_bytes(wv, tokens, cfg, ksl_opt);
 }
 

@@ -137,6 +137,8 @@ size_t sx_sk_bytes(const WeightView &wv, uint32_t tokens, int cfg, uint32_t ksl_
 // Whether the call takes the LDS-shared tiles (k_sxt); with cfg kSxUnshared none does.
 constexpr int kSxUnshared = -1;
 bool sx_shared(const WeightView &wv, uint32_t tokens, int cfg, uint32_t ksl_opt);
+// Whether launch_sx prepares x in a launch of its own.
+bool sx_prepares_x(const WeightView &wv, uint32_t tokens, int cfg, uint32_t ksl_opt);
 void sx_describe(const WeightView &wv, uint32_t tokens, int cfg, uint32_t ksl_opt, eff_split_plan_info *out);
 hipError_t launch_sx(const WeightView &wv, const float *x, float *y, uint32_t tokens, void *scratch, int cfg,
                      uint32_t ksl_opt, void *sk, hipStream_t stream);

@@ -106,9 +106,8 @@ typedef struct eff_stats {
                            router GEMM call, one per eff_gemm_prepare_x, one per eff_qmatmul_prepare_x
                            for the GEMM) */
   uint64_t split_x;     /* preparations of x for the split-x product in a launch of their own (one per
-                           split-x router call but those of Q2_K and IQ2_XXS up to 8 tokens under the
-                           automatic configuration, which prepare x inside the product; one per
-                           eff_qmatmul_prepare_x for it) */
+                           split-x router call but those of up to 8 tokens that prepare x inside the
+                           product: eff_split_plan's prepares_x; one per eff_qmatmul_prepare_x for it) */
   uint64_t cpu_path;    /* products with the reference CPU path's arithmetic (eff_qmatmul_cpu_path) */
 } eff_stats;
 

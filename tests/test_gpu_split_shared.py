@@ -224,15 +224,18 @@ def test_one_launch_in_k_slices(ctx, eff, orc, tname, rows, k, tokens):
     x[:256] *= 1e-3
     x[k:k + 256] *= 1e6
     wb = upload_w(ctx, eff, tname, data, n)
-    before = ctx.stats()["split"]
+    assert not eff.split_plan(t, rows, k, tokens)["prepares_x"]
+    before = ctx.stats()
     y = run(ctx, t, wb, x, rows, k, tokens)
-    assert ctx.stats()["split"] == before + 2
+    assert ctx.stats()["split"] == before["split"] + 2
+    assert ctx.stats()["split_x"] == before["split_x"]      # no preparation of its own: one launch
     ref = product(orc, "Q8_0" if tname == "Q8_0R" else tname, gguf, n, x, rows, k)
     assert (np.linalg.norm(y - ref, axis=1) <= REL * np.linalg.norm(ref, axis=1)).all()
     nb, _ = ctx.qmatmul_x_layout(t, rows, k, tokens)
     xb, xp, yb = ctx.upload(x), ctx.alloc(nb), ctx.alloc(tokens * rows * 4)
     ctx.qmatmul_prepare_x(t, xb, xp, rows, k, tokens)
     ctx.qmatmul_prepared(t, wb, xp, yb, rows, k, tokens)
+    assert ctx.stats()["split_x"] == before["split_x"] + 1
     assert np.array_equal(yb.read(np.uint32), y.view(np.uint32).ravel())
     for b in (wb, xb, xp, yb):
         b.free()

@@ -44,3 +44,13 @@ def test_split_plan_errors(eff):
     for none in (("Q4_K", 64, 256, 1), ("Q8_0", 64, 288, 64)):
         with pytest.raises(eff.NotApplicable):
             eff.split_plan(*none)
+
+
+def test_preparations_of_x(eff):
+    """x is prepared inside the product at up to 8 tokens of an automatic call with
+    few workgroups times k, and by a launch of its own everywhere else."""
+    for tname, rows, k, tokens, own in [("Q8_0", 2048, 8192, 8, 0), ("Q8_0R", 1024, 8192, 5, 0), ("Q6_K", 2048, 8192, 8, 0),
+                                        ("Q6_K", 4096, 14336, 8, 1), ("Q8_0", 2048, 8192, 9, 1), ("Q2_K", 8192, 2048, 6, 0),
+                                        ("IQ2_XXS", 65536, 2048, 5, 1), ("Q4_K", 4096, 4608, 8, 1), ("Q4_K", 8192, 2048, 512, 1)]:
+        assert eff.split_plan(tname, rows, k, tokens)["prepares_x"] == own, (tname, rows, k, tokens)
+        assert eff.split_plan(tname, rows, k, tokens, 1)["prepares_x"] == 1
