@@ -104,6 +104,13 @@ __device__ __forceinline__ void wait_vm() {
   __builtin_amdgcn_s_waitcnt((int)((N & 15u) | ((N >> 4) << 14) | 0x0F70u));
 }
 
+// Writes an output through L2 (agent scope): a tile's outputs leave at the end of
+// its workgroup, and what stays dirty in L2 is written back before the next launch
+// starts; written through they may stay in the memory-side cache for their reader,
+// which nontemporal stores keep them out of.
+__device__ __forceinline__ void store_through(float *o, float v) {
+  __hip_atomic_store(o, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 
 // Where the blocks of a weight tile live: `q` covers the GGUF blocks (or the
 // Q8_0R quants) from the tile's first block on, `s` the Q8_0R scales.

@@ -357,26 +357,19 @@ __global__ __launch_bounds__(kNW * 64) void k_gemm_q8(WeightView wv, const _Floa
   uint32_t lane_e;
   __asm__ volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(lane_e));
   const uint32_t ne = lane_e & 31u, he = lane_e >> 5;
-  // outputs v = 4 q .. 4 q + 3 of fragment (fi, fj), written through L2 (agent
-  // scope): a tile's outputs all leave at the end of its workgroup, and what
-  // stays dirty in L2 is written back before the next launch starts. Written
-  // through they may stay in the memory-side cache, which nontemporal stores keep
-  // them out of (us with the x conversion, plain / nontemporal / written through,
-  // y the same 67 MB each call and four of them in turn: 8192 x 2048 at 2048
-  // tokens 80.4 / 81.5 / 78.8 and 84.8 / 82.0 / 83.5; at 512 tokens 30.8 / 29.4 /
-  // 29.2 and 30.8 / 29.4 / 29.2)
-  auto store = [](float *o, float v) {
-    __hip_atomic_store(o, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  };
+  // outputs v = 4 q .. 4 q + 3 of fragment (fi, fj), written through L2 (us with
+  // the x conversion, plain / nontemporal / written through, y the same 67 MB each
+  // call and four of them in turn: 8192 x 2048 at 2048 tokens 80.4 / 81.5 / 78.8
+  // and 84.8 / 82.0 / 83.5; at 512 tokens 30.8 / 29.4 / 29.2 and 30.8 / 29.4 / 29.2)
   auto put = [&](int fi, int fj, int q, float4 v) {
     const uint32_t row = n0 + kFN * 32u * wn + 32u * (uint32_t)fj + ne;
     const uint32_t tok = t0 + kFM * 32u * wm + 32u * (uint32_t)fi + 8u * (uint32_t)q + 4u * he;
     if (row >= rows) return;
     float *o = y + (uint64_t)tok * rows + row;
-    if (tok < tokens) store(o, v.x);
-    if (tok + 1u < tokens) store(o + rows, v.y);
-    if (tok + 2u < tokens) store(o + 2ull * rows, v.z);
-    if (tok + 3u < tokens) store(o + 3ull * rows, v.w);
+    if (tok < tokens) store_through(o, v.x);
+    if (tok + 1u < tokens) store_through(o + rows, v.y);
+    if (tok + 2u < tokens) store_through(o + 2ull * rows, v.z);
+    if (tok + 3u < tokens) store_through(o + 3ull * rows, v.w);
   };
   auto mine = [&](int fi, int fj, int q) {
     return make_float4(acc[fi][fj][4 * q], acc[fi][fj][4 * q + 1], acc[fi][fj][4 * q + 2], acc[fi][fj][4 * q + 3]);
