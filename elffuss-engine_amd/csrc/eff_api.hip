@@ -342,7 +342,7 @@ int sk_scratch(eff_ctx *ctx, const WeightView &wv, uint32_t tokens, uint32_t pla
 
 // The k-slice scratch of a split-x product and the configuration it runs in.
 // The slices of the LDS-shared tiles have a buffer of their own, made with the
-// context at the largest size a plan of theirs has (42 MB): recorded or not,
+// context at the largest size a plan of theirs has (21 MB): recorded or not,
 // first call or later, a shape runs the same kernel and gives the same bits, and
 // no call frees what a recording reads. A context that found no memory for it
 // takes k_sx for those shapes, always.

@@ -828,9 +828,9 @@ __global__ __launch_bounds__(NW * 64) void k_sx(WeightView wv, const uint8_t *__
 // covers groups * tt tiles (tokens past `tokens` are zero).
 struct SxPlan {
   // cfg 0: 32 rows x 8 waves; 1: 64 rows x 4 waves; ksl: k slices per row tile;
-  // shared: the LDS-shared tiles (k_sxt) instead, their row tiles per wave, in ksl slices (0: k_sx)
+  // shared: the LDS-shared tiles (k_sxt) instead, in ksl slices
   uint32_t tt, cfg, groups, row_tiles, nbw, ksl;
-  uint32_t shared;
+  bool shared;
 };
 
 // The types folded per group of steps (Q8_0, Q8_0R, Q6_K) take at most 2
@@ -856,33 +856,28 @@ uint32_t sx_tile_count(int type, uint32_t tokens) {
   return tokens > 32u ? (tt * groups + 3u) / 4u * 4u : tt * groups;
 }
 
-// The row tiles (of 32 per wave: 1 or 2) and k slices of the LDS-shared tiles
-// (k_sxt) where they are estimated to be faster than the plan of k_sx, else 0.
-// Both times (us) are linear in a CU's rounds of workgroups and in the blocks of
-// k a round walks, plus the slices' sums; the coefficients are least-squares fits
-// (4-8% rms error) to timings of both kernels at 110 shapes a type from 1024 to
-// 14336 rows, k = 1024 to 8192 and 40 to 2048 tokens (k_sxt in 1 to 8 slices).
-// The choice is 0.1-0.4% above the faster of the two summed over them, and 22%
-// (Q4_K), 43% (Q6_K), 19% (Q2_K) and 10% (IQ2_XXS) below k_sx alone. us, k_sx /
-// k_sxt with one row tile / two: Q4_K 8192 x 2048 at 512 tokens 71 / 55 / 54, at
-// 256 36.8 / 29.9 / 36.4, 4096 x 4096 at 512 65.5 / 53.5 / 60.6, 1024 x 8192 at
-// 1000 87.6 / 63.8 / 68.9, but 4096 x 8192 at 128 37.8 / 35.4 / 42.2 and 2048 x
-// 2048 at 128 12.0 / 19.6 / 24.1; Q6_K 8192 x 2048 at 512 130 / 65, 2048 x 8192 at
-// 300 83 / 52 (3 slices), 2048 x 2048 at 128 13.0 / 17.0.
-uint32_t sxt_choose(const WeightView &wv, uint32_t tokens, double rounds, uint32_t walk, bool sliced, uint32_t &ksl) {
+// The k slices of the LDS-shared tiles (k_sxt) where they are estimated to be
+// faster than the plan of k_sx, else 0. Both times (us) are linear in a CU's rounds
+// of workgroups and in the blocks of k a round walks, plus the slices' sums; the
+// coefficients are least-squares fits (4-8% rms error) to timings of both kernels
+// (k_sxt in 1 to 8 slices) at 110 (Q2_K, Q6_K: 199) shapes a type. Over 199 shapes
+// (512 to 14336 rows, k = 1024 to 14336, 40 to 2048 tokens) the choice is 0.1-0.6%
+// above the faster of the two summed, at most 6% above k_sx (Q6_K 4096 x 2048 at 80
+// tokens), and 16% (Q4_K), 40% (Q6_K), 12% (Q2_K) and 12% (IQ2_XXS) below k_sx alone.
+// us, k_sx / k_sxt: Q4_K 8192 x 2048 at 512 tokens 72.1 / 56.4, at 300 49.8 / 48.7, at
+// 2048 261 / 221, 4096 x 4096 at 1500 185 / 150; Q6_K 8192 x 2048 at 512 130 / 71, but
+// 2048 x 4096 at 80 20.0 / 23.4 (8 slices).
+uint32_t sxt_choose(const WeightView &wv, uint32_t tokens, double rounds, uint32_t walk, bool sliced) {
   struct Fit {
     int type;
-    double sx[5];       // launch, per round, per round and block of a token tile, if sliced, per 1e6 values of x
-    double sxt[2][6];   // by row tiles: launch, per round, per round and pair of blocks, if sliced, per 1e6
-                        // sums of all slices, per 1e6 values of x (launch 0: not built)
+    double sx[5];    // launch, per round, per round and block of a token tile, if sliced, per 1e6 values of x
+    double sxt[6];   // launch, per round, per round and pair of blocks, if sliced, per 1e6 sums of all
+                     // slices, per 1e6 values of x
   };
-  static const Fit fits[] = {
-      {Q4_K, {4.30, 1.84, 0.209, 2.28, 3.42},
-       {{1.48, 6.22, 3.76, 2.20, 1.61, 3.78}, {0.17, 9.37, 6.90, 4.14, 1.84, 2.88}}},
-      {Q6_K, {4.30, 2.45, 0.356, 2.03, 3.07}, {{1.72, 5.62, 5.09, 1.80, 1.92, 3.29}, {0}}},
-      {Q2_K, {4.22, 1.57, 0.193, 2.16, 3.76},
-       {{2.15, 5.09, 3.57, 1.75, 1.62, 3.73}, {1.32, 7.92, 6.20, 2.70, 1.87, 3.07}}},
-      {IQ2_XXS, {4.78, 1.35, 0.189, 2.12, 3.68}, {{2.36, 5.06, 4.20, 1.76, 1.63, 3.26}, {0}}}};
+  static const Fit fits[] = {{Q4_K, {4.30, 1.84, 0.209, 2.28, 3.42}, {1.48, 6.22, 3.76, 2.20, 1.61, 3.78}},
+                             {Q6_K, {5.96, 2.71, 0.336, 1.68, 2.44}, {5.19, 6.14, 4.62, 0.38, 1.90, 2.43}},
+                             {Q2_K, {5.59, 1.72, 0.185, 2.04, 3.28}, {4.48, 4.69, 3.70, 1.48, 2.00, 2.63}},
+                             {IQ2_XXS, {4.78, 1.35, 0.189, 2.12, 3.68}, {2.36, 5.06, 4.20, 1.76, 1.63, 3.26}}};
   if (tokens <= 32u) return 0u;   // the x scratch then holds less than the kernel's 64 tokens
   const uint64_t nb = wv.k / 256u, xb = (uint64_t)sx_tile_count(wv.type, tokens) * nb * 17u * 1024u;
   if (xb >= (1ull << 32) || (uint64_t)wv.rows * nb * 210u >= (1ull << 32)) return 0u;   // 32-bit offsets
@@ -890,20 +885,17 @@ uint32_t sxt_choose(const WeightView &wv, uint32_t tokens, double rounds, uint32
     if (f.type != wv.type) continue;
     const double xk = 1e-6 * tokens * wv.k, out = 1e-6 * tokens * wv.rows;
     double best = 0.95 * (f.sx[0] + rounds * (f.sx[1] + f.sx[2] * walk) + (sliced ? f.sx[3] : 0.0) + f.sx[4] * xk);
-    uint32_t fb = 0u;
-    for (uint32_t i = 1u; i <= 2u; ++i) {
-      const double *c = f.sxt[i - 1u];
-      if (c[0] == 0.0) continue;
-      const uint64_t tiles = (uint64_t)((wv.rows + 128u * i - 1u) / (128u * i)) * ((tokens + 63u) / 64u);
-      for (uint32_t s : {1u, 2u, 3u, 4u, 6u, 8u}) {
-        if (s > 1u && (tiles * s > kSxtSliceWgs || nb / s < 2u)) break;
-        const uint64_t r = (tiles * s + 255u) / 256u, pairs = ((nb + s - 1u) / s + 1u) / 2u;
-        const double t = c[0] + (double)r * (c[1] + c[2] * (double)pairs) + (s > 1u ? c[3] + c[4] * out * s : 0.0) +
-                         c[5] * xk;
-        if (t < best) best = t, fb = i, ksl = s;
-      }
+    uint32_t ksl = 0u;
+    const double *c = f.sxt;
+    const uint64_t tiles = (uint64_t)((wv.rows + 127u) / 128u) * ((tokens + 63u) / 64u);
+    for (uint32_t s : {1u, 2u, 3u, 4u, 6u, 8u}) {
+      if (s > 1u && (tiles * s > kSxtSliceWgs || nb / s < 2u)) break;
+      const uint64_t r = (tiles * s + 255u) / 256u, pairs = ((nb + s - 1u) / s + 1u) / 2u;
+      const double t = c[0] + (double)r * (c[1] + c[2] * (double)pairs) + (s > 1u ? c[3] + c[4] * out * s : 0.0) +
+                       c[5] * xk;
+      if (t < best) best = t, ksl = s;
     }
-    return fb;
+    return ksl;
   }
   return 0u;
 }
@@ -955,14 +947,11 @@ SxPlan sx_plan(const WeightView &wv, uint32_t tokens, int cfg, uint32_t ksl_opt)
   p.nbw = ((nb + p.ksl - 1u) / p.ksl + nw - 1u) / nw;
   // the LDS-shared tiles, where they are estimated to be the faster
   const double rounds = p.ksl > 1u ? (p.cfg ? 1.75 : 1.0) * ((wgs * p.ksl + 255u) / 256u) : p.cfg ? t64 : t32;
-  uint32_t shared_ksl = 1u;
-  p.shared = share ? sxt_choose(wv, tokens, rounds, (nb + p.ksl - 1u) / p.ksl * p.tt, p.ksl > 1u, shared_ksl) : 0u;
-  if (p.shared) {
-    // a forced count whose sums the slices' buffer cannot hold stays on k_sx
-    const uint32_t ksl = max(1u, min(ksl_opt ? ksl_opt : shared_ksl, nb));
-    if (sxt_sk_bytes(wv, tokens, p.shared, ksl) <= kSxtSkBytes) p.ksl = ksl;
-    else p.shared = 0u;
-  }
+  const uint32_t sxt = share ? sxt_choose(wv, tokens, rounds, (nb + p.ksl - 1u) / p.ksl * p.tt, p.ksl > 1u) : 0u;
+  // a forced count whose sums the slices' buffer cannot hold stays on k_sx
+  const uint32_t sxt_ksl = max(1u, min(ksl_opt ? ksl_opt : sxt, nb));
+  p.shared = sxt && sxt_sk_bytes(wv, tokens, sxt_ksl) <= kSxtSkBytes;
+  if (p.shared) p.ksl = sxt_ksl;
   return p;
 }
 
@@ -1033,7 +1022,7 @@ template <int TYPE>
 hipError_t sx_main(const WeightView &wv, const uint8_t *xa, uint32_t tiles, float *y, uint32_t tokens,
                    const SxPlan &p, void *sk, hipStream_t s) {
   const float *xp = (const float *)(xa + (uint64_t)tiles * (wv.k / 256u) * sx_slots<TYPE>() * 1024u);
-  if (p.shared) return launch_sxt(wv, xa, xp, tiles, y, tokens, p.shared, p.ksl, sk, s);
+  if (p.shared) return launch_sxt(wv, xa, xp, tiles, y, tokens, p.ksl, sk, s);
   switch (p.tt) {
     case 1: return sx_cfg<TYPE, 1>(wv, xa, xp, y, tokens, p, sk, s);
     case 2: return sx_cfg<TYPE, 2>(wv, xa, xp, y, tokens, p, sk, s);
@@ -1083,14 +1072,14 @@ size_t sx_x_bytes(int type, uint32_t tokens, uint32_t k) {
 
 size_t sx_sk_bytes(const WeightView &wv, uint32_t tokens, int cfg, uint32_t ksl_opt) {
   const SxPlan p = sx_plan(wv, tokens, cfg, ksl_opt);
-  if (p.shared) return sxt_sk_bytes(wv, tokens, p.shared, p.ksl);
+  if (p.shared) return sxt_sk_bytes(wv, tokens, p.ksl);
   if (p.ksl < 2u || sx_fx(wv.type, tokens, cfg, p, wv.k)) return 0;
   const uint64_t ne = (uint64_t)p.tt * (p.cfg ? 2u : 1u) * 512u;   // sums per workgroup
   return kSliceCntBytes + (size_t)((uint64_t)p.row_tiles * p.groups * p.ksl * ne * 4u);
 }
 
 bool sx_shared(const WeightView &wv, uint32_t tokens, int cfg, uint32_t ksl_opt) {
-  return sx_plan(wv, tokens, cfg, ksl_opt).shared != 0u;
+  return sx_plan(wv, tokens, cfg, ksl_opt).shared;
 }
 
 bool sx_prepares_x(const WeightView &wv, uint32_t tokens, int cfg, uint32_t ksl_opt) {
@@ -1101,7 +1090,7 @@ bool sx_prepares_x(const WeightView &wv, uint32_t tokens, int cfg, uint32_t ksl_
 void sx_describe(const WeightView &wv, uint32_t tokens, int cfg, uint32_t ksl_opt, eff_split_plan_info *out) {
   const SxPlan p = sx_plan(wv, tokens, cfg, ksl_opt);
   out->shared = p.shared ? 1u : 0u;
-  out->rows = p.shared ? 128u * p.shared : p.cfg ? 64u : 32u;
+  out->rows = p.shared ? 128u : p.cfg ? 64u : 32u;
   out->slices = p.ksl;
   out->prepares_x = sx_prepares_x(wv, tokens, cfg, ksl_opt);
   out->slice_bytes = sx_sk_bytes(wv, tokens, cfg, ksl_opt);

@@ -8,42 +8,49 @@
 // clock and CU with the matrix cores busy, all that a CU's vector memory path
 // delivers. Here a workgroup's waves share x through LDS.
 //
-// Workgroup: 8 waves (2 per SIMD) over 64 tokens x 128 FB rows, as 4 groups of
-// 32 FB rows x 2 slices of k (slice z takes every second block of 256). A wave
-// holds 2 x FB tiles of 32 tokens x 32 rows: per step of 16 k it reads 2 lo and 2
-// hi fragments of x (4 KB) for 4 FB v_mfma_f32_32x32x16_f16, decodes its FB weight
-// fragments in registers, and adds lo and hi into one accumulator per tile,
-//   D += u lo, D += u hi,
-// folded once per block: acc += D d p (p: x's block scales). x flows in groups of 4 steps through two
-// LDS buffers (direct-to-LDS loads a group ahead, one barrier per group); the
-// raw weights of the next block are loaded into a region of LDS of the wave's
-// own while the present block's are in registers.
+// Workgroup: 8 waves (2 per SIMD) over 64 tokens x 128 rows, as 4 groups of 32
+// rows x 2 slices of k (slice z takes every second block of 256). A wave holds 2
+// tiles of 32 tokens x 32 rows: per step of 16 k it reads 2 lo and 2 hi fragments
+// of x (4 KB) for 4 v_mfma_f32_32x32x16_f16, decodes its weight fragment in
+// registers, and adds lo and hi into accumulators of their own,
+//   D2 += u lo, D += u hi,
+// folded once per block: acc += (D + D2) d p (p: x's block scales). x flows in
+// groups of 4 steps through two LDS buffers (direct-to-LDS loads a group ahead,
+// one barrier per group); the raw weights of the next block are loaded into a
+// region of LDS of the wave's own while the present block's are in registers.
 //
-// Errors against 64 bits are those of k_sx or smaller (2048 x 8192 to 8192 x
-// 2048, 300-512 tokens): a D that takes lo and hi parts is rounded twice as
-// often as one of the hi parts alone (1.25 times the error). Q4_K and Q2_K make
-// up for it with smaller sums: u = sc (q - 8) and sc (q - 1.5) instead of sc q,
-// and D opens with the group sums' terms, -(dmin / d) sum mn_g S_g + 8 (1.5)
-// sum sc_g S_g (1.9e-7 against 3.2e-7, 1.8e-7 against 2.1e-7). IQ2_XXS and Q6_K
-// keep the lo parts in accumulators of their own, which leaves registers for
-// one row tile per wave (FB = 1) (1.3e-7 as before; Q6_K 1.2e-7 against 1.7e-7, its hi
-// parts in two sums of 8 steps).
+// Errors against 64 bits are k_sx's or smaller, for weights of both signs and of
+// one (normal, |normal|, exponential and its cube, -|normal|, normal + 1 sigma) and
+// for x of both signs and of one, k = 512 to 14336. What it takes (relative L2, k =
+// 2048, normal x; k_sx / here):
+//  - Q4_K and Q2_K multiply u = sc (q - c) instead of sc q, c the block's zero as
+//    its minima put it (near dmin sum mn / (d sum sc): about half the range for
+//    weights of both signs, 0 where there are no minima), and D opens with the
+//    group sums' terms, -(dmin / d) sum mn_g S_g + c sum sc_g S_g: sums near those
+//    of the weights themselves. Normal weights 3.15e-7 / 1.46e-7 (Q4_K) and
+//    2.00e-7 / 1.42e-7 (Q2_K), |normal| 1.24e-7 / 1.04e-7 and 0.89e-7 / 0.84e-7, the
+//    cube of exponential 0.93e-7 / 0.86e-7 and 0.76e-7 / 0.76e-7. With c fixed at
+//    the middle of the range and lo in D, weights of one sign came to up to 4.5e-7.
+//  - A block's hi parts in two sums of 8 steps (not IQ2_XXS: 1.30e-7 both ways), the
+//    blocks in four runs.
+// A wave of 64 rows halves the reads of x, but with lo in accumulators of its own it
+// leaves registers for one wave per SIMD (us, Q4_K, 64 rows / 32: 8192 x 2048 at 512
+// tokens 57.8 / 58.2, at 1000 114.6 / 112.4, 4096 x 4096 at 1500 204 / 155), and its
+// error came to 1.1 of k_sx's for sums of one sign.
 //
 // Q6_K: u = sc (q - 32) has up to 13 bits, so its fp16 rounding v = fp16(u) is
 // off by r = u - v in {-1, 0, 1}, and only where |u| > 2048. The product takes
-// hi and lo times v plus hi times r; what is left out, lo times r, is below
-// 2^-22 of the term. Three matrix instructions instead of two, and one fold per
-// block instead of 16 (whose 24 vector instructions per matrix instruction
-// bound k_sx there).
+// hi and lo times v, hi times r, and, up to 8 blocks of k, lo times r (below 2^-22
+// of the term). Left out there it shows (1.00-1.08 of k_sx's error at k = 512 to
+// 2048, 0.96-1.01 with it); from 9 blocks the shorter chains of sums outweigh it
+// (0.87-0.91 at 3328, 0.71-0.73 at 8192). It costs a fourth matrix instruction
+// (8192 x 2048 at 512 tokens 62.9 / 69.7 us, k_sx 130). One fold per block instead of
+// 16, whose 24 vector instructions per matrix instruction bound k_sx there.
 //
-// What bounds it now: with random operands the matrix cores hold 1.4 PFLOP/s
-// beside 6 vector instructions per instruction (the clock falls from 2.4 to 1.5
-// GHz); a round of workgroups walks 512 k of 64 x 256 outputs per CU in 7 us
-// (Q4_K, 1.28 PFLOP/s of hi and lo products) after about 4 us for its first
-// loads, and ends with all of its y written at once, another 4. us, k_sx before
-// and this kernel, both with the preparation of x: Q4_K 8192 x 2048 at 512
-// tokens 63.8 / 48.8, Q6_K 2048 x 8192 at 300 78.0 / 50.0, Q4_K 4096 x 4096 at
-// 1000 125 / 91.
+// What bounds it: LDS reads, decode and matrix instructions of two waves per SIMD
+// in turn, after about 4 us of first loads. us, k_sx and this kernel, both with the
+// preparation of x: Q4_K 8192 x 2048 at 512 tokens 72.1 / 56.4, at 1000 150.0 / 107.2,
+// Q6_K 2048 x 8192 at 300 78.0 / 50.4.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>
@@ -93,15 +100,25 @@ __device__ __forceinline__ void min_ratio(float &d, float dm, float &ratio) {
   d = d != 0.f ? d : dm;
 }
 
+// The sum of a word's bytes, added to `acc`.
+__device__ __forceinline__ uint32_t bytes_sum(uint32_t w, uint32_t acc) {
+  return __builtin_amdgcn_udot4(w, 0x01010101u, acc, false);
+}
+
+// Of 0 .. most, the nearest to ratio mn / sc (0 where that is no number): where the
+// block's zero lies, in units of the type's steps for it.
+__device__ __forceinline__ float centre_of(float ratio, uint32_t mn, uint32_t sc, float most) {
+  return fminf(fmaxf(rintf(ratio * (float)mn * __builtin_amdgcn_rcpf((float)sc)), 0.f), most);
+}
+
 // Q4_K, 144 bytes: d | dmin | scales[12] | qs[128]. Piece 0: the header; pieces
 // 1 + 2 c + m: qs of 64-weight chunk c, bytes 16 m .. (piece 9 is the next
 // block's and not read).
 template <> struct SxtW<Q4_K> {
   static constexpr uint32_t NI = 5, UNITS = 1, BB = 144;
   static constexpr bool REM = false;
-  static constexpr bool SEP = false;
   uint32_t q[16], sc[2], mi[2];
-  float d, ratio;
+  float d, ratio, mid;
   __device__ static void fetch(rsrc_t src, const uint8_t *reg, uint32_t voff, uint32_t bo, int, uint32_t h) {
 #pragma unroll
     for (uint32_t i = 0; i < NI; ++i) dma16(src, reg + 1024u * i, voff + 16u * h, bo + 32u * i);
@@ -121,18 +138,20 @@ template <> struct SxtW<Q4_K> {
     sc[1] = ((hd.w & 0x0F0F0F0Fu) | ((hd.y >> 2) & 0x30303030u)) & keep;
     mi[1] = ((hd.w >> 4) & 0x0F0F0F0Fu) | ((hd.z >> 2) & 0x30303030u);
     min_ratio(d, 32.f * h2f(hd.x >> 16), ratio);  // group sums are stored divided by 32
+    mid = 4.f * centre_of(-0.0078125f * ratio, bytes_sum(mi[0], bytes_sum(mi[1], 0u)),
+                          bytes_sum(sc[0], bytes_sum(sc[1], 0u)), 3.f);
   }
-  // u = sc (q - 8), from the nibble in a byte's high half: (1024 + 16 q) sc / 16 - 72 sc
+  // u = sc (q - c), from the nibble in a byte's high half: (1024 + 16 q) sc / 16 - (64 + c) sc, c 0, 4, 8 or 12
   __device__ half8 step(int s, uint32_t, const uint8_t *) const {
     const int c = s >> 2, nib = (s >> 1) & 1, m = s & 1;
     const uint32_t w0 = q[4 * c + 2 * m], w1 = q[4 * c + 2 * m + 1];
     return dec_centred((nib ? w0 : w0 << 4) & 0xF0F0F0F0u, (nib ? w1 : w1 << 4) & 0xF0F0F0F0u,
-                       byte_of(sc, (uint32_t)s >> 1), 0.0625f, -72.f);
+                       byte_of(sc, (uint32_t)s >> 1), 0.0625f, -64.f - mid);
   }
   // 8 minima and 8 scales: one instruction takes the sums' hi parts in k 0..7, lo in 8..15
   static constexpr uint32_t MSTEP = 1;
   __device__ half8 mins(uint32_t) const { return dec_plain(mi[0], mi[1]); }
-  __device__ half8 centre(uint32_t) const { return dec_plain(sc[0], sc[1]) * (_Float16)256.f; }   // 8 x 32 sc
+  __device__ half8 centre(uint32_t) const { return dec_plain(sc[0], sc[1]) * (_Float16)(32.f * mid); }
 };
 
 // Q2_K, 84 bytes: scales[16] | qs[64] | d | dmin. Pieces 0: scales, 1 + 2 n + m:
@@ -140,9 +159,8 @@ template <> struct SxtW<Q4_K> {
 template <> struct SxtW<Q2_K> {
   static constexpr uint32_t NI = 3, UNITS = 1, BB = 84;
   static constexpr bool REM = false;
-  static constexpr bool SEP = false;
   uint32_t q[8], sc[4];
-  float d, ratio;
+  float d, ratio, mid;
   __device__ static void fetch(rsrc_t src, const uint8_t *reg, uint32_t voff, uint32_t bo, int, uint32_t h) {
 #pragma unroll
     for (uint32_t i = 0; i < NI; ++i) dma16(src, reg + 1024u * i, voff + 16u * h, bo + 32u * i);
@@ -160,21 +178,28 @@ template <> struct SxtW<Q2_K> {
       q[2 * p + 1] = (uint32_t)(v >> 32);
     }
     min_ratio(d, 16.f * h2f(w >> 16), ratio);  // group sums are stored divided by 16
+    uint32_t m = 0u, t = 0u;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      m = bytes_sum((sc[i] >> 4) & 0x0F0F0F0Fu, m);
+      t = bytes_sum(sc[i] & 0x0F0F0F0Fu, t);
+    }
+    mid = 0.5f * centre_of(-0.125f * ratio, m, t, 6.f);
   }
-  // u = sc (q - 1.5), from the 2 bits at a byte's top: (1024 + 64 q) sc / 64 - 17.5 sc
+  // u = sc (q - c), from the 2 bits at a byte's top: (1024 + 64 q) sc / 64 - (16 + c) sc, c 0, 0.5 .. 3
   __device__ half8 step(int s, uint32_t, const uint8_t *) const {
     const int n = s >> 3, g = (s >> 1) & 3, m = s & 1;
     return dec_centred((q[4 * n + 2 * m] << (6 - 2 * g)) & 0xC0C0C0C0u,
                        (q[4 * n + 2 * m + 1] << (6 - 2 * g)) & 0xC0C0C0C0u, byte_of(sc, (uint32_t)s) & 15u, 0.015625f,
-                       -17.5f);
+                       -16.f - mid);
   }
   static constexpr uint32_t MSTEP = 2;   // 16 minima: lo, then hi
   __device__ half8 mins(uint32_t h) const {
     const uint32_t w0 = h ? sc[2] : sc[0], w1 = h ? sc[3] : sc[1];
     return dec_plain((w0 >> 4) & 0x0F0F0F0Fu, (w1 >> 4) & 0x0F0F0F0Fu);
   }
-  __device__ half8 centre(uint32_t h) const {   // 1.5 x 16 sc
-    return dec_plain((h ? sc[2] : sc[0]) & 0x0F0F0F0Fu, (h ? sc[3] : sc[1]) & 0x0F0F0F0Fu) * (_Float16)24.f;
+  __device__ half8 centre(uint32_t h) const {
+    return dec_plain((h ? sc[2] : sc[0]) & 0x0F0F0F0Fu, (h ? sc[3] : sc[1]) & 0x0F0F0F0Fu) * (_Float16)(16.f * mid);
   }
 };
 
@@ -186,7 +211,6 @@ template <> struct SxtW<Q2_K> {
 template <> struct SxtW<IQ2_XXS> {
   static constexpr uint32_t NI = 3, UNITS = 1, BB = 66;
   static constexpr bool REM = false;
-  static constexpr bool SEP = true;
   uint32_t g[8], sc;   // g[i]: steps 2 i and 2 i + 1, 16 bits each: index | field << 8
   float d, ratio;
   __device__ static void fetch(rsrc_t src, const uint8_t *reg, uint32_t voff, uint32_t bo, int, uint32_t h) {
@@ -240,7 +264,6 @@ template <> struct SxtW<IQ2_XXS> {
 template <> struct SxtW<Q6_K> {
   static constexpr uint32_t NI = 5, UNITS = 2, BB = 210;
   static constexpr bool REM = true;
-  static constexpr bool SEP = true;
   uint32_t ql[8], qh[4], sc[2];
   float d, ratio;
   __device__ static void fetch(rsrc_t src, const uint8_t *reg, uint32_t voff, uint32_t bo, int un, uint32_t h) {
@@ -302,17 +325,17 @@ __device__ __forceinline__ void wait_vm_lds() {
 }
 
 constexpr uint32_t kTokTile = 64;    // tokens per workgroup: 4 tiles of 16 of the prepared x
+constexpr uint32_t kSxtLorBlocks = 8;    // Q6_K: blocks of k up to which lo times r is taken too
 
-// FB: tiles of 32 rows per wave, a workgroup having 4 groups of 32 FB rows.
-template <int TYPE, int FB>
+template <int TYPE>
 struct SxtLds {
   static constexpr uint32_t XG = 2u * 4u * 4096u;                   // 4 steps of 64 tokens, for each k slice
   static constexpr uint32_t WR = SxtW<TYPE>::NI * 1024u;            // raw weights of 32 rows
   static constexpr uint32_t TAB = TYPE == IQ2_XXS ? 2048u : 0u;
-  static constexpr uint32_t X0 = TAB, W0 = X0 + 2u * XG, M0 = W0 + 8u * FB * WR;
+  static constexpr uint32_t X0 = TAB, W0 = X0 + 2u * XG, M0 = W0 + 8u * WR;
   static constexpr uint32_t P0 = M0 + (sx_mins<TYPE>() ? 8192u : 0u);   // group sums of a block, for each k slice
   static constexpr uint32_t LOOP = P0 + 1024u;                      // block scales: 2 blocks x 2 slices x 64 tokens
-  static constexpr uint32_t RED = 8u * 8192u + 16u;                 // the waves' sums handed over
+  static constexpr uint32_t RED = 8u * 4096u + 16u;                 // the waves' sums handed over
   static constexpr uint32_t BYTES = LOOP > RED ? LOOP : RED;
   static_assert(BYTES <= 160u * 1024u, "LDS");
 };
@@ -321,19 +344,21 @@ __device__ __forceinline__ float16v mma(half8 a, half8 b, float16v c) {
   return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
 }
 
-template <int TYPE, int FB>
+// LOR: lo times r as well (Q6_K)
+template <int TYPE, bool LOR>
 __global__ __launch_bounds__(512) void k_sxt(WeightView wv, const uint8_t *__restrict__ xa,
                                              const float *__restrict__ xp, float *__restrict__ y, uint32_t tokens,
                                              uint32_t xa_bytes, uint32_t xp_bytes, uint32_t row_tiles,
                                              uint32_t tok_tiles, uint32_t ksl, float *__restrict__ part,
                                              uint32_t *__restrict__ cnt) {
   using W = SxtW<TYPE>;
-  using L = SxtLds<TYPE, FB>;
+  using L = SxtLds<TYPE>;
   constexpr bool MINS = sx_mins<TYPE>();
+  constexpr bool HALF = MINS || W::REM;          // a block's hi parts in two sums of 8 steps
   constexpr uint32_t NS = sx_slots<TYPE>();
-  static_assert(FB == 1 || (FB == 2 && !W::SEP), "registers");
+  static_assert(!LOR || W::REM, "r");
   constexpr uint32_t SU = 16u / W::UNITS;        // steps of a unit
-  constexpr uint32_t WI = FB * W::NI;            // a wave's loads of a unit's weights
+  constexpr uint32_t WI = W::NI;                 // a wave's loads of a unit's weights
   constexpr uint32_t XI = 4u;                    // and of a group's x
   __shared__ __align__(16) uint8_t lds[L::BYTES];
   const uint32_t tid = threadIdx.x, lane = tid & 63u, j = lane & 31u, h = lane >> 5;
@@ -345,7 +370,7 @@ __global__ __launch_bounds__(512) void k_sxt(WeightView wv, const uint8_t *__res
   uint32_t u = blockIdx.x;
   if (nwg % 8u == 0u) u = (blockIdx.x % 8u) * (nwg / 8u) + blockIdx.x / 8u;
   const uint32_t z = u / ntiles, lin = u - z * ntiles;
-  const uint32_t tt0 = lin % tok_tiles, r0 = (lin / tok_tiles) * (128u * FB) + 32u * FB * rg;
+  const uint32_t tt0 = lin % tok_tiles, r0 = (lin / tok_tiles) * 128u + 32u * rg;
   const uint32_t rows = wv.rows, nb = wv.k / 256u;
   const uint32_t bl = z * nb / ksl, bh = (z + 1u) * nb / ksl, iters = (bh - bl + 1u) / 2u;
 
@@ -354,21 +379,14 @@ __global__ __launch_bounds__(512) void k_sxt(WeightView wv, const uint8_t *__res
   }
 
   const rsrc_t wsrc = make_rsrc(wv.w, wv.w_bytes), xsrc = make_rsrc(xa, xa_bytes), psrc = make_rsrc(xp, xp_bytes);
-  const uint32_t rb = (uint32_t)wv.row_bytes;
-  uint32_t wrow[FB];
-#pragma unroll
-  for (int f = 0; f < FB; ++f) wrow[f] = min(r0 + 32u * f + j, rows - 1u) * rb;
-  uint8_t *const wreg = lds + L::W0 + wave * FB * L::WR;
+  const uint32_t wrow = min(r0 + j, rows - 1u) * (uint32_t)wv.row_bytes;
+  uint8_t *const wreg = lds + L::W0 + wave * L::WR;
   const uint32_t pvoff = ((4u * tt0 + (lane >> 4)) * nb * 16u + (lane & 15u)) * 4u;
   const uint32_t xtile = (4u * tt0 + (wave & 3u)) * nb;
 
   // the block of slice sl in iteration it (loads past the end repeat the last block)
   auto blk = [&](uint32_t it, uint32_t sl) { return min(bl + 2u * it + sl, bh - 1u); };
-  auto fetch_w = [&](uint32_t it, int un) {
-    const uint32_t b = blk(it, ks);
-#pragma unroll
-    for (int f = 0; f < FB; ++f) W::fetch(wsrc, wreg + f * L::WR, wrow[f], b * W::BB, un, h);
-  };
+  auto fetch_w = [&](uint32_t it, int un) { W::fetch(wsrc, wreg, wrow, blk(it, ks) * W::BB, un, h); };
   // x of group g (4 steps) of iteration it: 1 KB chunk c = wave + 8 i is
   // 16-token tile c % 4 of step c / 4 % 4 of slice c / 16
   auto fetch_x = [&](uint32_t it, uint32_t g) {
@@ -388,19 +406,24 @@ __global__ __launch_bounds__(512) void k_sxt(WeightView wv, const uint8_t *__res
   // the lane's fragment rows: token j of a tile of 32 = row j % 16 of 16-token tile j / 16
   const uint8_t *const xl = lds + L::X0 + ks * 16384u + (j >> 4) * 1024u + 16u * (32u * h + (j & 15u));
 
-  // [token tile][row tile]; D2: the sums of the lo parts (and of hi times r)
-  // where they are kept apart
-  float16v acc[2][FB], D[2][FB], D2[2][W::SEP ? FB : 1], E[2][W::REM ? FB : 1];
+  // by token tile of 32. D: a block's sums of the hi parts (HALF: of its second
+  // half, E holding the first's), D2: of the lo parts and of the products with r;
+  // acc: the folded sums of a run of blocks, total: of the runs before it
+  float16v total[2], acc[2], D[2], D2[2], E[HALF ? 2 : 1];
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+  for (int a = 0; a < 2; ++a) total[a] = acc[a] = float16v{};
+  auto end_run = [&]() {
 #pragma unroll
-    for (int f = 0; f < FB; ++f) acc[a][f] = float16v{};
+    for (int a = 0; a < 2; ++a) {
+#pragma unroll
+      for (int v = 0; v < 16; ++v) total[a][v] += acc[a][v];
+      acc[a] = float16v{};
+    }
+  };
 
-  W w[FB];
+  W w;
   auto take_w = [&](uint32_t it, int un) {
-    const uint32_t bo = blk(it, ks) * W::BB;
-#pragma unroll
-    for (int f = 0; f < FB; ++f) w[f].take(wreg + f * L::WR, un, j, h, (wrow[f] + bo) & 2u);
+    w.take(wreg, un, j, h, (wrow + blk(it, ks) * W::BB) & 2u);
     // every read of the region has returned before the next loads into it go out
     __asm__ volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   };
@@ -412,73 +435,53 @@ __global__ __launch_bounds__(512) void k_sxt(WeightView wv, const uint8_t *__res
     for (int a = 0; a < 2; ++a) A[q][a] = *(const half8 *)(p + 2048 * a);
     __asm__ volatile("" ::: "memory");
   };
-  half8 B[2][FB], R[2][W::REM ? FB : 1];
+  half8 B[2], R[2];
   auto decode = [&](uint32_t set, uint32_t s) {
-#pragma unroll
-    for (int f = 0; f < FB; ++f) {
-      if constexpr (W::REM) B[set][f] = w[f].step2((int)(s % SU), R[set][f]);
-      else B[set][f] = w[f].step((int)s, h, lds);
-    }
+    if constexpr (W::REM) B[set] = w.step2((int)(s % SU), R[set]);
+    else B[set] = w.step((int)s, h, lds);
   };
   auto low = [&](uint32_t set) {
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-      for (int f = 0; f < FB; ++f) {
-        float16v &d = W::SEP ? D2[a][W::SEP ? f : 0] : D[a][f];
-        d = mma(A[1][a], B[set][f], d);
-      }
+    for (int a = 0; a < 2; ++a) {
+      D2[a] = mma(A[1][a], B[set], D2[a]);
+      if constexpr (LOR) D2[a] = mma(A[1][a], R[set], D2[a]);
+    }
   };
   auto high = [&](uint32_t set) {
 #pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-      for (int f = 0; f < FB; ++f) D[a][f] = mma(A[0][a], B[set][f], D[a][f]);
+    for (int a = 0; a < 2; ++a) D[a] = mma(A[0][a], B[set], D[a]);
     if constexpr (W::REM) {
 #pragma unroll
-      for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int f = 0; f < FB; ++f) D2[a][f] = mma(A[0][a], R[set][f], D2[a][f]);
+      for (int a = 0; a < 2; ++a) D2[a] = mma(A[0][a], R[set], D2[a]);
     }
   };
-  // D at the start of a block: the minima's sums, scaled, and the centres'
-  float dcur[FB];
+  // D at the start of a block: the minima's sums, scaled, and the centre's
+  float dcur;
   auto open = [&]() {
+#pragma unroll
+    for (int a = 0; a < 2; ++a) D[a] = D2[a] = float16v{};
     if constexpr (MINS) {
-      const uint8_t *ml = lds + L::M0 + ks * 4096u + (j >> 4) * 1024u + 16u * ((W::MSTEP == 1u ? 16u : 32u) * h + (j & 15u));
+      const uint8_t *ml =
+          lds + L::M0 + ks * 4096u + (j >> 4) * 1024u + 16u * ((W::MSTEP == 1u ? 16u : 32u) * h + (j & 15u));
       half8 ms[2][W::MSTEP];
 #pragma unroll
       for (int a = 0; a < 2; ++a)
 #pragma unroll
         for (uint32_t q = 0; q < W::MSTEP; ++q) ms[a][q] = *(const half8 *)(ml + 2048 * a + 256u * q);
+      const half8 mb = w.mins(h), cb = w.centre(h);
 #pragma unroll
-      for (int f = 0; f < FB; ++f) {
-        const half8 mb = w[f].mins(h), cb = w[f].centre(h);
+      for (int a = 0; a < 2; ++a)
 #pragma unroll
-        for (int a = 0; a < 2; ++a) {
-          D[a][f] = float16v{};
+        for (int q = (int)W::MSTEP - 1; q >= 0; --q) D[a] = mma(ms[a][q], mb, D[a]);
 #pragma unroll
-          for (int q = (int)W::MSTEP - 1; q >= 0; --q) D[a][f] = mma(ms[a][q], mb, D[a][f]);
+      for (int a = 0; a < 2; ++a) {
 #pragma unroll
-          for (int v = 0; v < 16; ++v) D[a][f][v] *= w[f].ratio;
+        for (int v = 0; v < 16; ++v) D[a][v] *= w.ratio;
 #pragma unroll
-          for (int q = (int)W::MSTEP - 1; q >= 0; --q) D[a][f] = mma(ms[a][q], cb, D[a][f]);
-        }
+        for (int q = (int)W::MSTEP - 1; q >= 0; --q) D[a] = mma(ms[a][q], cb, D[a]);
       }
-    } else {
-#pragma unroll
-      for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int f = 0; f < FB; ++f) D[a][f] = float16v{};
     }
-    if constexpr (W::SEP) {
-#pragma unroll
-      for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int f = 0; f < FB; ++f) D2[a][f] = float16v{};
-    }
-#pragma unroll
-    for (int f = 0; f < FB; ++f) dcur[f] = w[f].d;
+    dcur = w.d;
   };
 
   // prologue: the first unit's weights, the first block's sums and scales, x of
@@ -495,158 +498,152 @@ __global__ __launch_bounds__(512) void k_sxt(WeightView wv, const uint8_t *__res
   read_a(0, 0u, 0u);
   decode(0u, 0u);
 
-  for (uint32_t it = 0; it < iters; ++it) {
-    open();
+  // more than 12 blocks in runs of a quarter of them: as many partial sums as the
+  // waves of k_sx make (one run of 28 blocks: 1.1 of k_sx's error for sums of one
+  // sign; the runs cost 1-2% of the time at 4 to 8 blocks, where one is as exact)
+  const uint32_t run = iters > 12u ? (iters + 3u) / 4u : iters;
+  for (uint32_t it = 0; it < iters;) {
+    for (const uint32_t end = min(it + run, iters); it < end; ++it) {
+      open();
 #pragma unroll
-    for (uint32_t s = 0; s < 16u; ++s) {
-      const uint32_t cur = s & 1u, nxt = cur ^ 1u, g = s >> 2, gn = (g + ((s & 3u) == 3u)) & 3u, sn = (s + 1u) & 3u;
-      // lo parts; at a group's end, between the two, the next group's x is in
-      // LDS once every wave's own loads of it are (a group ago; the weights of
-      // the next unit went out after them), and the present group's buffer is
-      // free once every wave has read it
-      if constexpr (W::REM)
-        if (s == 8u) {
+      for (uint32_t s = 0; s < 16u; ++s) {
+        const uint32_t cur = s & 1u, nxt = cur ^ 1u, g = s >> 2, gn = (g + ((s & 3u) == 3u)) & 3u, sn = (s + 1u) & 3u;
+        if constexpr (HALF)
+          if (s == 8u) {
 #pragma unroll
-          for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int f = 0; f < FB; ++f) {
-              E[a][f] = D[a][f];
-              D[a][f] = float16v{};
+            for (int a = 0; a < 2; ++a) {
+              E[a] = D[a];
+              D[a] = float16v{};
             }
+          }
+        // lo parts; at a group's end, between the two, the next group's x is in
+        // LDS once every wave's own loads of it are (a group ago; the weights of
+        // the next unit went out after them), and the present group's buffer is
+        // free once every wave has read it
+        low(cur);
+        if ((s & 3u) == 3u) {
+          __builtin_amdgcn_sched_barrier(0);
+          if (g % (W::UNITS == 1u ? 4u : 2u) == 0u) wait_vm_lds<WI>();
+          else wait_vm_lds<0>();
+          __builtin_amdgcn_s_barrier();
+          __asm__ volatile("" ::: "memory");
+          if (g == 2u) fetch_m(it + 1u);
+          fetch_x(g < 2u ? it : it + 1u, (g + 2u) & 3u);
         }
-      low(cur);
-      if ((s & 3u) == 3u) {
+        read_a(1, gn, sn);
+        if ((s + 1u) % SU == 0u) {
+          // the next unit: its weights into registers, and the loads of the one after
+          const uint32_t ni = s == 15u ? it + 1u : it;
+          const int un = s == 15u ? 0 : 1;
+          take_w(ni, un);
+          fetch_w(un + 1 == (int)W::UNITS ? ni + 1u : ni, un + 1 == (int)W::UNITS ? 0 : un + 1);
+        }
+        // hi parts, while the next step's weights are decoded
+        decode(nxt, (s + 1u) & 15u);
+        high(cur);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
+        }
+        read_a(0, gn, sn);
         __builtin_amdgcn_sched_barrier(0);
-        if (g % (W::UNITS == 1u ? 4u : 2u) == 0u) wait_vm_lds<WI>();
-        else wait_vm_lds<0>();
-        __builtin_amdgcn_s_barrier();
-        __asm__ volatile("" ::: "memory");
-        if (g == 2u) fetch_m(it + 1u);
-        fetch_x(g < 2u ? it : it + 1u, (g + 2u) & 3u);
       }
-      read_a(1, gn, sn);
-      if ((s + 1u) % SU == 0u) {
-        // the next unit: its weights into registers, and the loads of the one after
-        const uint32_t ni = s == 15u ? it + 1u : it;
-        const int un = s == 15u ? 0 : 1;
-        take_w(ni, un);
-        fetch_w(un + 1 == (int)W::UNITS ? ni + 1u : ni, un + 1 == (int)W::UNITS ? 0 : un + 1);
-      }
-      // hi parts, while the next step's weights are decoded
-      decode(nxt, (s + 1u) & 15u);
-      high(cur);
+      // the fold
+      if (bl + 2u * it + ks < bh) {
+        const uint8_t *pp = lds + L::P0 + (it & 1u) * 512u + ks * 256u + 16u * h;
 #pragma unroll
-      for (int i = 0; i < 4 * FB; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-        __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);
-      }
-      read_a(0, gn, sn);
-      __builtin_amdgcn_sched_barrier(0);
-    }
-    // the fold
-    if (bl + 2u * it + ks < bh) {
-      const uint8_t *pp = lds + L::P0 + (it & 1u) * 512u + ks * 256u + 16u * h;
+        for (int a = 0; a < 2; ++a)
 #pragma unroll
-      for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const float4 p = *(const float4 *)(pp + 128 * a + 32 * g);
-#pragma unroll
-          for (int f = 0; f < FB; ++f)
+          for (int g = 0; g < 4; ++g) {
+            const float4 p = *(const float4 *)(pp + 128 * a + 32 * g);
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-              float t = D[a][f][4 * g + v];
-              if constexpr (W::REM) t = E[a][f][4 * g + v] + t;
-              if constexpr (W::SEP) t += D2[a][f][4 * g + v];
-              acc[a][f][4 * g + v] =
-                  __builtin_fmaf(t * dcur[f], v == 0 ? p.x : v == 1 ? p.y : v == 2 ? p.z : p.w, acc[a][f][4 * g + v]);
+              float t = D[a][4 * g + v] + D2[a][4 * g + v];
+              if constexpr (HALF) t += E[a][4 * g + v];
+              acc[a][4 * g + v] =
+                  __builtin_fmaf(t * dcur, v == 0 ? p.x : v == 1 ? p.y : v == 2 ? p.z : p.w, acc[a][4 * g + v]);
             }
-        }
+          }
+      }
     }
+    end_run();
   }
   wait_vm<0>();
   __syncthreads();
 
-  // the two k slices' sums, slice 0 + slice 1: a wave writes 32 FB tokens x 32
-  // rows of its row group (two row tiles: tile ks, one: token tile ks) and hands
-  // the rest over in LDS
+  // the two k slices' sums, slice 0 + slice 1: a wave writes token tile ks of its
+  // 32 rows and hands the other over in LDS
   float *const red = (float *)lds;
-  float16v sum[FB];
+  float16v sum;
 #pragma unroll
-  for (int i = 0; i < FB; ++i)
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const float a0 = acc[i][0][v], a1 = FB == 2 ? acc[i][FB - 1][v] : acc[1][0][v];
-      sum[i][v] = ks ? a1 : a0;
-      red[((wave * FB + i) * 16u + v) * 64u + lane] = ks ? a0 : a1;
-    }
+  for (int v = 0; v < 16; ++v) {
+    sum[v] = ks ? total[1][v] : total[0][v];
+    red[(wave * 16u + v) * 64u + lane] = ks ? total[0][v] : total[1][v];
+  }
   __syncthreads();
 #pragma unroll
-  for (int i = 0; i < FB; ++i)
-#pragma unroll
-    for (int v = 0; v < 16; ++v) sum[i][v] += red[(((wave ^ 4u) * FB + i) * 16u + v) * 64u + lane];
+  for (int v = 0; v < 16; ++v) sum[v] += red[((wave ^ 4u) * 16u + v) * 64u + lane];
 
   if (ksl > 1u) {
     // k slices over workgroups, as in eff_gemm_sx.hip: the last of the tile's
-    // ksl workgroups to arrive adds the slices in slice order
+    // ksl workgroups to arrive adds the slices, two by two, the pairs in order (all in
+    // a row, sums of one sign over 6 slices came to 1.06 of k_sx's error)
     constexpr int kSc1 = 16;   // cache policy bit 4: sc1
-    constexpr uint32_t NE = kTokTile * 128u * FB;
+    constexpr uint32_t NE = kTokTile * 128u;
     uint32_t *const arrived = (uint32_t *)(lds + L::BYTES - 16u);
     const rsrc_t prs = make_rsrc(part + (uint64_t)lin * ksl * NE, (uint64_t)ksl * NE * 4u);
-    auto off = [&](uint32_t zz, uint32_t a, uint32_t v4) {
-      return (int)(zz * (NE * 4u) + (((wave * FB + a) * 4u + v4) * 64u + lane) * 16u);
+    auto off = [&](uint32_t zz, uint32_t v4) {
+      return (int)(zz * (NE * 4u) + ((wave * 4u + v4) * 64u + lane) * 16u);
     };
 #pragma unroll
-    for (uint32_t a = 0; a < (uint32_t)FB; ++a)
-#pragma unroll
-      for (uint32_t v = 0; v < 4u; ++v) {
-        const u32x4 o = {__float_as_uint(sum[a][4 * v]), __float_as_uint(sum[a][4 * v + 1]),
-                         __float_as_uint(sum[a][4 * v + 2]), __float_as_uint(sum[a][4 * v + 3])};
-        __builtin_amdgcn_raw_buffer_store_b128(o, prs, off(z, a, v), 0, kSc1);
-      }
+    for (uint32_t v = 0; v < 4u; ++v) {
+      const u32x4 o = {__float_as_uint(sum[4 * v]), __float_as_uint(sum[4 * v + 1]), __float_as_uint(sum[4 * v + 2]),
+                       __float_as_uint(sum[4 * v + 3])};
+      __builtin_amdgcn_raw_buffer_store_b128(o, prs, off(z, v), 0, kSc1);
+    }
     __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();   // every wave's sums are stored
     if (tid == 0u) *arrived = __hip_atomic_fetch_add(cnt + lin, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
     if (*arrived != ksl - 1u) return;
     if (tid == 0u) __hip_atomic_store(cnt + lin, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    for (uint32_t zz = 0; zz < ksl; ++zz) {
+    for (uint32_t zz = 0; zz < ksl; zz += 2u) {
+      const bool two = zz + 1u < ksl;
 #pragma unroll
-      for (uint32_t a = 0; a < (uint32_t)FB; ++a)
+      for (uint32_t v = 0; v < 4u; ++v) {
+        const u32x4 o = __builtin_amdgcn_raw_buffer_load_b128(prs, off(zz, v), 0, kSc1);
+        const u32x4 q = __builtin_amdgcn_raw_buffer_load_b128(prs, off(two ? zz + 1u : zz, v), 0, kSc1);
 #pragma unroll
-        for (uint32_t v = 0; v < 4u; ++v) {
-          const u32x4 o = __builtin_amdgcn_raw_buffer_load_b128(prs, off(zz, a, v), 0, kSc1);
-#pragma unroll
-          for (int c = 0; c < 4; ++c)
-            sum[a][4 * v + c] = zz ? sum[a][4 * v + c] + __uint_as_float(o[c]) : __uint_as_float(o[c]);
+        for (int c = 0; c < 4; ++c) {
+          const float t = two ? __uint_as_float(o[c]) + __uint_as_float(q[c]) : __uint_as_float(o[c]);
+          sum[4 * v + c] = zz ? sum[4 * v + c] + t : t;
         }
+      }
     }
   }
   // written through L2 (us, plain / nontemporal / written through, and with the next
   // layer's product, which reads y: Q4_K 8192 x 2048 at 512 tokens 50.6 / 49.0 / 49.1
   // and 104.3 / 104.0 / 102.7, Q6_K 2048 x 8192 at 300 53.5 / 52.0 / 51.4 and 93.5 /
   // 91.6 / 91.0)
-  const uint32_t row = r0 + (FB == 2 ? 32u * ks : 0u) + j;
+  const uint32_t row = r0 + j;
   if (row >= rows) return;
 #pragma unroll
-  for (uint32_t a = 0; a < (uint32_t)FB; ++a)
-#pragma unroll
-    for (uint32_t v = 0; v < 16u; ++v) {
-      const uint32_t tok = kTokTile * tt0 + 32u * (FB == 2 ? a : ks) + 8u * (v >> 2) + 4u * h + (v & 3u);
-      if (tok < tokens) store_through(y + (uint64_t)tok * rows + row, sum[a][v]);
-    }
+  for (uint32_t v = 0; v < 16u; ++v) {
+    const uint32_t tok = kTokTile * tt0 + 32u * ks + 8u * (v >> 2) + 4u * h + (v & 3u);
+    if (tok < tokens) store_through(y + (uint64_t)tok * rows + row, sum[v]);
+  }
 }
 
 struct SxtPlan {
   uint32_t row_tiles, tok_tiles, ksl;
 };
 
-SxtPlan sxt_plan(const WeightView &wv, uint32_t tokens, uint32_t fb, uint32_t ksl) {
-  return {(wv.rows + 128u * fb - 1u) / (128u * fb), (tokens + kTokTile - 1u) / kTokTile,
-          (uint32_t)max(1u, min(ksl, wv.k / 256u))};
+SxtPlan sxt_plan(const WeightView &wv, uint32_t tokens, uint32_t ksl) {
+  return {(wv.rows + 127u) / 128u, (tokens + kTokTile - 1u) / kTokTile, (uint32_t)max(1u, min(ksl, wv.k / 256u))};
 }
 
-template <int TYPE, int FB>
+template <int TYPE>
 hipError_t sxt_go(const WeightView &wv, const uint8_t *xa, const float *xp, uint32_t tiles, float *y,
                   uint32_t tokens, const SxtPlan &p, void *sk, hipStream_t s) {
   const uint64_t nb = wv.k / 256u, xb = (uint64_t)tiles * nb * sx_slots<TYPE>() * 1024u;
@@ -654,36 +651,31 @@ hipError_t sxt_go(const WeightView &wv, const uint8_t *xa, const float *xp, uint
   if (p.ksl > 1u && (!sk || (uint64_t)p.row_tiles * p.tok_tiles > kSliceCntBytes / 4u)) return hipErrorInvalidValue;
   uint32_t *cnt = (uint32_t *)sk;
   float *part = sk ? (float *)((uint8_t *)sk + kSliceCntBytes) : nullptr;
-  hipLaunchKernelGGL((k_sxt<TYPE, FB>), dim3(p.row_tiles * p.tok_tiles * p.ksl), dim3(512), 0, s, wv, xa, xp, y,
-                     tokens, (uint32_t)xb, (uint32_t)(tiles * nb * 64u), p.row_tiles, p.tok_tiles, p.ksl, part, cnt);
+  constexpr bool REM = SxtW<TYPE>::REM;
+  auto *const kernel = REM && nb <= kSxtLorBlocks ? k_sxt<TYPE, REM> : k_sxt<TYPE, false>;
+  hipLaunchKernelGGL(kernel, dim3(p.row_tiles * p.tok_tiles * p.ksl), dim3(512), 0, s, wv, xa, xp, y, tokens,
+                     (uint32_t)xb, (uint32_t)(tiles * nb * 64u), p.row_tiles, p.tok_tiles, p.ksl, part, cnt);
   return hipGetLastError();
 }
 
 }  // namespace
 
-size_t sxt_sk_bytes(const WeightView &wv, uint32_t tokens, uint32_t fb, uint32_t ksl) {
-  const SxtPlan p = sxt_plan(wv, tokens, fb, ksl);
+size_t sxt_sk_bytes(const WeightView &wv, uint32_t tokens, uint32_t ksl) {
+  const SxtPlan p = sxt_plan(wv, tokens, ksl);
   if (p.ksl < 2u) return 0;
-  return kSliceCntBytes + (size_t)p.row_tiles * p.tok_tiles * p.ksl * (kTokTile * 128u * fb * 4u);
+  return kSliceCntBytes + (size_t)p.row_tiles * p.tok_tiles * p.ksl * (kTokTile * 128u * 4u);
 }
 
 hipError_t launch_sxt(const WeightView &wv, const void *xa, const void *xp, uint32_t tiles, float *y,
-                      uint32_t tokens, uint32_t fb, uint32_t ksl, void *sk, hipStream_t s) {
-  const SxtPlan p = sxt_plan(wv, tokens, fb, ksl);
+                      uint32_t tokens, uint32_t ksl, void *sk, hipStream_t s) {
+  const SxtPlan p = sxt_plan(wv, tokens, ksl);
   const uint8_t *a = (const uint8_t *)xa;
   const float *b = (const float *)xp;
-  if (fb == 2u) {
-    switch (wv.type) {
-      case Q4_K: return sxt_go<Q4_K, 2>(wv, a, b, tiles, y, tokens, p, sk, s);
-      case Q2_K: return sxt_go<Q2_K, 2>(wv, a, b, tiles, y, tokens, p, sk, s);
-      default: return hipErrorInvalidValue;
-    }
-  }
   switch (wv.type) {
-    case Q4_K: return sxt_go<Q4_K, 1>(wv, a, b, tiles, y, tokens, p, sk, s);
-    case Q6_K: return sxt_go<Q6_K, 1>(wv, a, b, tiles, y, tokens, p, sk, s);
-    case Q2_K: return sxt_go<Q2_K, 1>(wv, a, b, tiles, y, tokens, p, sk, s);
-    case IQ2_XXS: return sxt_go<IQ2_XXS, 1>(wv, a, b, tiles, y, tokens, p, sk, s);
+    case Q4_K: return sxt_go<Q4_K>(wv, a, b, tiles, y, tokens, p, sk, s);
+    case Q6_K: return sxt_go<Q6_K>(wv, a, b, tiles, y, tokens, p, sk, s);
+    case Q2_K: return sxt_go<Q2_K>(wv, a, b, tiles, y, tokens, p, sk, s);
+    case IQ2_XXS: return sxt_go<IQ2_XXS>(wv, a, b, tiles, y, tokens, p, sk, s);
     default: return hipErrorInvalidValue;
   }
 }

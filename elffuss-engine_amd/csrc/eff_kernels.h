@@ -157,17 +157,17 @@ hipError_t launch_sx_prepared(const WeightView &wv, const void *xprep, float *y,
                               uint32_t ksl_opt, void *sk, hipStream_t stream);
 
 // The split-x product over LDS-shared tiles (eff_gemm_sxt.hip; Q2_K, Q4_K,
-// IQ2_XXS, Q6_K): 64 tokens x 128 fb rows per workgroup (fb 1; 2 also for Q2_K
-// and Q4_K), k in ksl slices over workgroups; x prepared for `tiles` token tiles
-// of 16 (a multiple of 4, xp the tokens' block scales).
-size_t sxt_sk_bytes(const WeightView &wv, uint32_t tokens, uint32_t fb, uint32_t ksl);
+// IQ2_XXS, Q6_K): 64 tokens x 128 rows per workgroup, k in ksl slices over
+// workgroups; x prepared for `tiles` token tiles of 16 (a multiple of 4, xp the
+// tokens' block scales).
+size_t sxt_sk_bytes(const WeightView &wv, uint32_t tokens, uint32_t ksl);
 // Automatic k slices keep within 640 workgroups; the scratch they then take at
-// most (64 tokens x 256 rows of sums each), and what a context holds for them: a
+// most (64 tokens x 128 rows of sums each), and what a context holds for them: a
 // forced count that would need more takes k_sx.
 constexpr uint32_t kSxtSliceWgs = 640u;
-constexpr size_t kSxtSkBytes = kSliceCntBytes + (size_t)kSxtSliceWgs * 64u * 256u * 4u;
+constexpr size_t kSxtSkBytes = kSliceCntBytes + (size_t)kSxtSliceWgs * 64u * 128u * 4u;
 hipError_t launch_sxt(const WeightView &wv, const void *xa, const void *xp, uint32_t tiles, float *y,
-                      uint32_t tokens, uint32_t fb, uint32_t ksl, void *sk, hipStream_t stream);
+                      uint32_t tokens, uint32_t ksl, void *sk, hipStream_t stream);
 
 // The reference CPU path's arithmetic for Q8_0 (eff_cpu_path.hip): x into
 // 40-byte 8-bit blocks in `act` (cpu_path_act_bytes(...)), then per row and

@@ -71,7 +71,7 @@ extern "C" {
                                        take none); the slices' sums are added in slice order, so each count
                                        gives fixed bits */
 #define EFF_OPT_SPLIT_SLICES     8  /* split-x product, k slices over workgroups (tuning): 0 automatic (default),
-                                       else that many (1: none); the slices' sums are added in slice order */
+                                       else that many (1: none); the slices' sums are added in a fixed order */
 
 /* ---- fused GEMV modes (gemv2Shader `modo`, kernels.gemv.wgsl.js:370-375) -- */
 #define EFF_GEMV_SECTIONS  1  /* 'secciones': ys[i] = W_i x for 2..4 matrices */
@@ -128,7 +128,7 @@ int eff_type_geometry(int type, uint32_t *block_elems, uint32_t *block_bytes);
 /* ---- context -------------------------------------------------------------- */
 
 /* Open a context on HIP device `device` with its own stream (default priority) and
- * 42 MB of device memory for the k slices of the split-x prompts; where that cannot
+ * 21 MB of device memory for the k slices of the split-x prompts; where that cannot
  * be had, the context runs those without slices.
  * Replaces requestDevice + createOps (device.js:66-139, ops.js:1604-1633). */
 int eff_init(int device, eff_ctx **out);

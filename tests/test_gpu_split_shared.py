@@ -15,13 +15,15 @@ pytestmark = pytest.mark.gpu
 # them stay under 16 ulp (2^-20) of the output's norm
 REL = 2.0 ** -20
 
-# (type, rows, k, tokens): shapes at which the planner takes the shared tiles, of
-# one and (Q4_K, Q2_K) two row tiles per wave, whole and in 2 to 8 k slices
-SHAPES = [("Q4_K", 513, 256, 4000), ("Q4_K", 1000, 4352, 1000), ("Q4_K", 513, 8192, 501), ("Q4_K", 777, 768, 4000),
-          ("Q4_K", 3000, 2304, 449), ("Q4_K", 700, 4352, 1500), ("Q2_K", 513, 256, 4000),
-          ("Q2_K", 513, 8192, 501), ("Q2_K", 3000, 768, 1000),
-          ("Q6_K", 1000, 256, 520), ("Q6_K", 777, 768, 1000), ("Q6_K", 513, 2304, 1000), ("Q6_K", 1000, 8192, 65),
-          ("IQ2_XXS", 777, 256, 2000), ("IQ2_XXS", 513, 4352, 501)]
+# (type, rows, k, tokens): shapes at which the planner takes the shared tiles (held
+# to that by test_shapes_take_the_shared_tiles), whole and in 2 to 8 k slices; Q6_K
+# also up to 8 blocks of k, where it takes one product more
+SHAPES = [("Q4_K", 641, 256, 2000), ("Q4_K", 1000, 4352, 1000), ("Q4_K", 513, 8192, 501), ("Q4_K", 777, 768, 4000),
+          ("Q4_K", 3000, 2304, 449), ("Q4_K", 700, 4352, 1500), ("Q2_K", 641, 256, 2000),
+          ("Q2_K", 513, 8192, 501), ("Q2_K", 777, 768, 4000),
+          ("Q6_K", 1500, 256, 777), ("Q6_K", 777, 768, 1000), ("Q6_K", 513, 2304, 1000), ("Q6_K", 1000, 8192, 65),
+          ("IQ2_XXS", 777, 256, 2000), ("IQ2_XXS", 513, 4352, 501), ("Q2_K", 1000, 4352, 1000),
+          ("Q6_K", 513, 2048, 1000)]
 
 
 def product(orc, tname, gguf, n, x, rows, k):
@@ -38,6 +40,13 @@ def run(ctx, t, wb, x, rows, k, tokens):
     xb.free(); yb.free()
     assert np.array_equal(y.view(np.uint32), again.view(np.uint32))   # whatever the order of arrival
     return y
+
+
+def test_shapes_take_the_shared_tiles(eff):
+    plans = [eff.split_plan(*s) for s in SHAPES]
+    assert all(p["shared"] for p in plans)
+    assert {1, 2, 3, 6, 8} <= {p["slices"] for p in plans}
+    assert not any(eff.split_plan(*s, 1)["shared"] for s in SHAPES)
 
 
 @pytest.mark.parametrize("tname,rows,k,tokens", SHAPES)
@@ -98,6 +107,56 @@ def test_shared_tiles_range_and_non_finite(ctx, eff, orc, tname, rows, k, tokens
     wb.free()
 
 
+# weights of one sign and of both: Q4_K and Q2_K then hold no minima, or minima only
+WEIGHTS = {"normal": lambda z, e: z, "abs": lambda z, e: np.abs(z), "exp3": lambda z, e: e ** 3,
+           "neg": lambda z, e: -np.abs(z)}
+PROMPTS = [(1000, 512, 777), (1024, 2048, 1000), (513, 8192, 501)]
+
+
+@pytest.mark.parametrize("tname,rows,k,tokens", [(t, *s) for t in ("Q4_K", "Q2_K", "Q6_K") for s in PROMPTS])
+@pytest.mark.parametrize("positive_x", [False, True])
+def test_error_no_larger_than_the_other_kernels(ctx, eff, orc, tname, rows, k, tokens, positive_x):
+    """Relative L2 error against 64 bits beside that of the kernel whose waves read x
+    by themselves, for weights of both signs and of one. The two add the same terms in
+    another order, which by itself moves the error by up to 2%: 1.05 of it at most."""
+    assert eff.split_plan(tname, rows, k, tokens)["shared"]
+    t = eff.TYPES[tname]
+    x = eff.fill_normal(76, 1.0, tokens * k)
+    x = np.abs(x) if positive_x else x
+    z = eff.fill_normal(75, 0.02, rows * k)
+    e = np.abs(eff.fill_normal(77, 0.2, rows * k))
+    for kind, f in WEIGHTS.items():
+        data = eff.quantize(t, np.ascontiguousarray(f(z, e), np.float32))
+        ref = product(orc, tname, data, rows * k // 256, x, rows, k)
+        wb = ctx.upload(data)
+        err = []
+        try:
+            for cfg in (0, 1):
+                ctx.set_option(eff.OPT_SPLIT_CONFIG, cfg)
+                err.append(np.linalg.norm(run(ctx, t, wb, x, rows, k, tokens) - ref) / np.linalg.norm(ref))
+        finally:
+            ctx.set_option(eff.OPT_SPLIT_CONFIG, 0)
+            wb.free()
+        print(f"{tname} {rows}x{k} M={tokens} {kind}: {err[0]:.3e} beside {err[1]:.3e}", flush=True)
+        assert err[0] <= 1.05 * err[1], kind
+
+
+@pytest.mark.parametrize("tname", ["Q4_K", "Q2_K"])
+def test_zero_weights_give_zero(ctx, eff, tname):
+    """Blocks whose quants and minima are zero, at scales that are not: every output
+    is 0, as the sums of the weights themselves are."""
+    rows, k, tokens = 1000, 512, 777
+    assert eff.split_plan(tname, rows, k, tokens)["shared"]
+    data = np.zeros((rows * k // 256, 144 if tname == "Q4_K" else 84), np.uint8)
+    if tname == "Q4_K":
+        data[:, 1], data[:, 3], data[:, 4:8] = 0x20, 0x20, 63      # d, dmin and the first scales
+    else:
+        data[:, :16], data[:, 81], data[:, 83] = 15, 0x20, 0x20
+    wb = ctx.upload(data)
+    assert not run(ctx, eff.TYPES[tname], wb, eff.fill_normal(5, 1.0, tokens * k), rows, k, tokens).any()
+    wb.free()
+
+
 def test_recorded_before_any_eager_call_gives_the_eager_bits(eff, orc):
     """A shape whose shared tiles take k slices, recorded in a context in which no
     eager call has taken them: the recording runs the same kernel, gives the bits of
@@ -152,7 +211,7 @@ def test_recorded_before_any_eager_call_gives_the_eager_bits(eff, orc):
 
 def test_forced_slices_leave_a_recording_its_buffer(eff, orc):
     """A recording of the sliced shared tiles, then eager calls whose forced slice
-    count needs more than the slices' buffer holds (256 tiles x 8): they run the
+    count needs more than the slices' buffer holds (512 tiles x 8): they run the
     other kernel, and the recording replays its bits."""
     with eff.Context(0) as ctx:
         small, big = ("Q6_K", 2048, 8192, 300), ("Q4_K", 8192, 2048, 512)
@@ -162,7 +221,8 @@ def test_forced_slices_leave_a_recording_its_buffer(eff, orc):
         for tname, rows, k, tokens in (small, big):
             t, data, gguf, n = make_weights(eff, tname, rows, k, 97)
             x = eff.fill_normal(98, 1.0, tokens * k)
-            st.append((t, ctx.upload(data), ctx.upload(x), ctx.alloc(tokens * rows * 4), product(orc, tname, gguf, n, x, rows, k)))
+            st.append((t, ctx.upload(data), ctx.upload(x), ctx.alloc(tokens * rows * 4),
+                       product(orc, tname, gguf, n, x, rows, k)))
         t, wb, xb, yb, ref = st[0]
         t2, wb2, xb2, yb2, ref2 = st[1]
         ctx.qmatmul(t2, wb2, xb2, yb2, *big[1:])

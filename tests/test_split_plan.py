@@ -3,8 +3,8 @@ from the shape, the type and the options alone, so checked without a device."""
 import pytest
 
 # what a context holds for the k slices of the LDS-shared tiles: the tiles'
-# counters and the sums of 640 workgroups of 64 tokens x 256 rows
-SLICE_BUFFER = (1 << 18) + 640 * 64 * 256 * 4
+# counters and the sums of 640 workgroups of 64 tokens x 128 rows
+SLICE_BUFFER = (1 << 18) + 640 * 64 * 128 * 4
 
 ROWS = [1, 130, 513, 1024, 2048, 4096, 8192, 14336, 32768]
 TOKENS = [33, 64, 65, 129, 300, 512, 1000, 2048, 5000]
@@ -31,7 +31,7 @@ def test_shared_tiles_never_need_more_than_their_buffer(eff, tname):
                     if slices:
                         assert p["slices"] == min(slices, k // 256)
     assert seen > 100 and turned_away > 50
-    # 256 tiles in 8 slices: 134 MB
+    # 512 tiles in 8 slices: 134 MB
     if tname == "Q4_K":
         assert not eff.split_plan("Q4_K", 8192, 2048, 512, 0, 8)["shared"]
         assert eff.split_plan("Q4_K", 8192, 2048, 512)["shared"]
@@ -49,8 +49,10 @@ def test_split_plan_errors(eff):
 def test_preparations_of_x(eff):
     """x is prepared inside the product at up to 8 tokens of an automatic call with
     few workgroups times k, and by a launch of its own everywhere else."""
-    for tname, rows, k, tokens, own in [("Q8_0", 2048, 8192, 8, 0), ("Q8_0R", 1024, 8192, 5, 0), ("Q6_K", 2048, 8192, 8, 0),
-                                        ("Q6_K", 4096, 14336, 8, 1), ("Q8_0", 2048, 8192, 9, 1), ("Q2_K", 8192, 2048, 6, 0),
-                                        ("IQ2_XXS", 65536, 2048, 5, 1), ("Q4_K", 4096, 4608, 8, 1), ("Q4_K", 8192, 2048, 512, 1)]:
+    for tname, rows, k, tokens, own in [("Q8_0", 2048, 8192, 8, 0), ("Q8_0R", 1024, 8192, 5, 0),
+                                        ("Q6_K", 2048, 8192, 8, 0), ("Q6_K", 4096, 14336, 8, 1),
+                                        ("Q8_0", 2048, 8192, 9, 1), ("Q2_K", 8192, 2048, 6, 0),
+                                        ("IQ2_XXS", 65536, 2048, 5, 1), ("Q4_K", 4096, 4608, 8, 1),
+                                        ("Q4_K", 8192, 2048, 512, 1)]:
         assert eff.split_plan(tname, rows, k, tokens)["prepares_x"] == own, (tname, rows, k, tokens)
         assert eff.split_plan(tname, rows, k, tokens, 1)["prepares_x"] == 1
