@@ -81,6 +81,8 @@ struct eff_ctx {
   void *sk_scratch = nullptr;       // k-slice counters and sums (GEMM and split-x)
   size_t sk_scratch_bytes = 0;
   void *sxt_scratch = nullptr;      // the same of the LDS-shared split-x tiles, kSxtSkBytes (sx_slices)
+  bool recorded = false;            // launches may have been recorded into a graph that outlives them
+  std::vector<void *> kept;         // scratch buffers replaced since then (grow)
   hipEvent_t order_ev = nullptr;    // orders a newly set stream after the previous one
   int64_t sx_min_tokens = 0;        // 0: the measured default (sx_routes)
   void *act_scratch = nullptr;      // x in the CPU path's 8-bit blocks (eff_qmatmul_cpu_path)
@@ -301,7 +303,10 @@ int run_gemv(eff_ctx *ctx, const WeightView &wv, const float *x, float *y, uint3
 }
 
 // Grow a context-owned scratch buffer (outside of any graph capture: the
-// first call of a shape must be eager).
+// first call of a shape must be eager). Where a recording may hold the present
+// one (ctx->recorded) it is kept until eff_shutdown instead of being freed, and
+// the new one is at least twice its size, so that all that is kept stays below
+// the size in use.
 int grow(eff_ctx *ctx, void **p, size_t *have, size_t need, const char *what) {
   if (need <= *have) return EFF_OK;
   hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
@@ -309,14 +314,21 @@ int grow(eff_ctx *ctx, void **p, size_t *have, size_t need, const char *what) {
   if (cs != hipStreamCaptureStatusNone)
     return fail(ctx, EFF_E_INVALID, "%s scratch of %zu bytes: it cannot grow while the stream is recorded into a "
                 "graph; run the largest call of this shape once before the recording", what, need);
-  if (*p) {
+  if (*p && !ctx->recorded) {
     EFF_HIP(ctx, hipStreamSynchronize(ctx->stream));
     (void)hipFree(*p);
     *p = nullptr;
     *have = 0;
   }
-  if (hipMalloc(p, need) != hipSuccess) return fail(ctx, EFF_E_NOMEM, "%s scratch of %zu bytes", what, need);
-  *have = need;
+  size_t size = *p && need < 2 * *have ? 2 * *have : need;
+  void *q = nullptr;
+  if (hipMalloc(&q, size) != hipSuccess && (size == need || hipMalloc(&q, size = need) != hipSuccess)) {
+    (void)hipGetLastError();
+    return fail(ctx, EFF_E_NOMEM, "%s scratch of %zu bytes", what, need);
+  }
+  if (*p) ctx->kept.push_back(*p);
+  *p = q;
+  *have = size;
   return EFF_OK;
 }
 
@@ -543,6 +555,7 @@ int eff_shutdown(eff_ctx *ctx) {
   if (ctx->act_scratch) (void)hipFree(ctx->act_scratch);
   if (ctx->sk_scratch) (void)hipFree(ctx->sk_scratch);
   if (ctx->sxt_scratch) (void)hipFree(ctx->sxt_scratch);
+  for (void *p : ctx->kept) (void)hipFree(p);
   if (ctx->order_ev) (void)hipEventDestroy(ctx->order_ev);
   for (auto &p : ctx->stage_pend) (void)hipEventDestroy(p.ev);
   for (hipEvent_t ev : ctx->events) (void)hipEventDestroy(ev);
@@ -555,7 +568,11 @@ int eff_shutdown(eff_ctx *ctx) {
 
 const char *eff_last_error(const eff_ctx *ctx) { return ctx ? ctx->error.c_str() : "no context"; }
 
-void *eff_stream(eff_ctx *ctx) { return ctx ? (void *)ctx->stream : nullptr; }
+void *eff_stream(eff_ctx *ctx) {
+  if (!ctx) return nullptr;
+  ctx->recorded = true;   // the caller may record what runs on it
+  return (void *)ctx->stream;
+}
 
 // The context's scratch buffers (and the k-slice counters, which must be
 // zero when a launch starts) are reused by every call, so a call on the new
@@ -578,6 +595,7 @@ int eff_set_stream(eff_ctx *ctx, void *hip_stream) {
     EFF_HIP(ctx, hipStreamWaitEvent(next, ctx->order_ev, 0));
   }
   ctx->stream = next;
+  if (next != ctx->own) ctx->recorded = true;   // the caller may record what runs on it
   return EFF_OK;
 }
 
@@ -1380,6 +1398,7 @@ int eff_graph_begin(eff_ctx *ctx) {
   // thread-local: only calls from this thread that could not be recorded
   // (waits, allocations) are refused while recording
   EFF_HIP(ctx, hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
+  ctx->recorded = true;
   return EFF_OK;
 }
 

@@ -175,7 +175,8 @@ int eff_get_stats(const eff_ctx *ctx, eff_stats *out);
  * eff_buf_free, eff_buf_retire, eff_buf_write, eff_buf_write_r, eff_buf_read,
  * eff_read_begin, and an op whose scratch would have to grow) return
  * EFF_E_INVALID and leave the recording open. An op's scratch is grown by
- * its first call of a shape outside a recording. */
+ * its first call of a shape outside a recording; the memory a recording uses
+ * stays allocated until eff_shutdown, also when a later call grows it. */
 int eff_graph_begin(eff_ctx *ctx);
 int eff_graph_end(eff_ctx *ctx, eff_graph **out);
 int eff_graph_launch(eff_ctx *ctx, eff_graph *g);

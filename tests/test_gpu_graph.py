@@ -79,6 +79,50 @@ def _refused_while_recording(ctx, eff):
         b.free()
 
 
+def test_recording_outlives_the_growth_of_its_scratch(eff):
+    """Products recorded at small sizes (split-x with its k slices, the GEMM with
+    its, the top-k), then eager calls that grow every scratch buffer they use, and
+    buffers allocated and filled after that: the recording replays its bits."""
+    with eff.Context(0) as ctx:
+        rows, k = 2048, 8192
+        ws = {t: ctx.upload(eff.quantize(t, eff.fill_normal(41, 0.02, rows * k))) for t in ("Q4_K", "Q8_0")}
+        x = ctx.upload(eff.fill_normal(42, 1.0, 600 * k))
+        y = ctx.alloc(600 * rows * 4)
+        logits = ctx.upload(eff.fill_normal(43, 1.0, 1 << 20))
+        out = ctx.alloc(eff.lib().eff_topk_out_bytes())
+        ys = [ctx.alloc(n * rows * 4) for n in (16, 64)]
+        small = [("Q4_K", 16), ("Q8_0", 64)]
+
+        def chain():
+            for (t, n), yb in zip(small, ys):
+                ctx.qmatmul(t, ws[t], x, yb, rows, k, n)
+            ctx.topk(logits, 0, 5000, 40, serial=3, out=out)
+
+        def read():
+            return [b.read(np.uint32) for b in ys + [out]]
+
+        chain()
+        want = read()
+        ctx.graph_begin()
+        chain()
+        g = ctx.graph_end()
+        for n in (130, 300, 600):
+            for t in ws:
+                ctx.qmatmul(t, ws[t], x, y, rows, k, n)
+        ctx.topk(logits, 0, 1 << 20, 40, serial=3, out=out)
+        junk = [ctx.upload(np.full(1 << 22, 0x7F7F7F7F, np.uint32)) for _ in range(8)]
+        for _ in range(3):
+            for b in ys + [out]:
+                b.write(np.zeros(b.size // 4, np.uint32))
+            g.launch()
+            for a, b in zip(read(), want):
+                assert np.array_equal(a, b)
+            ctx.qmatmul("Q4_K", ws["Q4_K"], x, y, rows, k, 600)
+        g.destroy()
+        for b in [*ws.values(), x, y, logits, out, *ys, *junk]:
+            b.free()
+
+
 def test_retire_is_stream_ordered(ctx, eff):
     """A weight buffer given back right after a product is enqueued, and a new
     buffer of the same size filled with other weights at once: the product
