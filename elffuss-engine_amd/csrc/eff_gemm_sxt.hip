@@ -35,8 +35,8 @@
 //    blocks in four runs.
 // A wave of 64 rows halves the reads of x, but with lo in accumulators of its own it
 // leaves registers for one wave per SIMD (us, Q4_K, 64 rows / 32: 8192 x 2048 at 512
-// tokens 57.8 / 58.2, at 1000 114.6 / 112.4, 4096 x 4096 at 1500 204 / 155), and its
-// error came to 1.1 of k_sx's for sums of one sign.
+// tokens 53.8 / 54.6, at 2048 206 / 230, 14336 x 4096 at 512 177 / 170): 0.4% over 199
+// shapes.
 //
 // Q6_K: u = sc (q - 32) has up to 13 bits, so its fp16 rounding v = fp16(u) is
 // off by r = u - v in {-1, 0, 1}, and only where |u| > 2048. The product takes
@@ -47,10 +47,12 @@
 // (8192 x 2048 at 512 tokens 62.9 / 69.7 us, k_sx 130). One fold per block instead of
 // 16, whose 24 vector instructions per matrix instruction bound k_sx there.
 //
-// What bounds it: LDS reads, decode and matrix instructions of two waves per SIMD
-// in turn, after about 4 us of first loads. us, k_sx and this kernel, both with the
-// preparation of x: Q4_K 8192 x 2048 at 512 tokens 72.1 / 56.4, at 1000 150.0 / 107.2,
-// Q6_K 2048 x 8192 at 300 78.0 / 50.4.
+// What bounds it: no unit (Q4_K 8192 x 2048 at 512 tokens: matrix cores busy 37% of
+// the kernel's clocks at 1.9 GHz, vector instructions 40%, LDS 27%, L2 10 TB/s). A CU
+// holds one workgroup, and nothing covers its first loads (about 4 us), the barrier
+// per group, the chain at a block's start and its end. us, k_sx and this kernel, both
+// with the preparation of x: Q4_K 8192 x 2048 at 512 tokens 72.1 / 56.4, at 1000 150.0 /
+// 107.2, Q6_K 2048 x 8192 at 300 78.0 / 50.4.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include <stdint.h>

@@ -425,9 +425,9 @@ __global__ __launch_bounds__(256) void k_gather(WeightView wv, const uint32_t *_
 // that the lanes' 16-byte stores spread over the banks), and leaves it in whole
 // lines, 16 bytes per lane: written to x by the decoding lanes, 16 bytes of each
 // 128-byte line at a time, and summed through LDS in 8 barriers, 700 tokens of
-// 2048 (Q6_K) took 7.0 us, now 5.0 (8192 x 64, Q8_0: 8.9 and 5.1); what is left is one chain (id, block,
-// decode, sum) per workgroup and the launch. The squares are summed per thread
-// over its columns, then across the workgroup in a fixed order.
+// 2048 (Q6_K) took 6.6 us, now 4.8 (8192 x 64, Q8_0: 8.9 and 5.1); what is left is
+// one chain (id, block, decode, sum) per workgroup and the launch. The squares are
+// summed per thread over its columns, then across the workgroup in a fixed order.
 __device__ __forceinline__ uint32_t gn_at(uint32_t c) { return c + (c >> 5) * 4u; }
 
 template <int TYPE>
