@@ -144,6 +144,7 @@ template <> struct SxtW<Q4_K> {
                           bytes_sum(sc[0], bytes_sum(sc[1], 0u)), 3.f);
   }
   // u = sc (q - c), from the nibble in a byte's high half: (1024 + 16 q) sc / 16 - (64 + c) sc, c 0, 4, 8 or 12
+  // (multiples of 4: (64 + c) sc, up to 4788, is exact in fp16)
   __device__ half8 step(int s, uint32_t, const uint8_t *) const {
     const int c = s >> 2, nib = (s >> 1) & 1, m = s & 1;
     const uint32_t w0 = q[4 * c + 2 * m], w1 = q[4 * c + 2 * m + 1];
