@@ -35,8 +35,7 @@
 //    blocks in four runs.
 // A wave of 64 rows halves the reads of x, but with lo in accumulators of its own it
 // leaves registers for one wave per SIMD (us, Q4_K, 64 rows / 32: 8192 x 2048 at 512
-// tokens 53.8 / 54.6, at 2048 206 / 230, 14336 x 4096 at 512 177 / 170): 0.4% over 199
-// shapes.
+// tokens 53.8 / 54.6, 14336 x 4096 at 512 177 / 170): 0.4% over 199 shapes.
 //
 // Q6_K: u = sc (q - 32) has up to 13 bits, so its fp16 rounding v = fp16(u) is
 // off by r = u - v in {-1, 0, 1}, and only where |u| > 2048. The product takes
@@ -328,6 +327,7 @@ __device__ __forceinline__ void wait_vm_lds() {
 }
 
 constexpr uint32_t kTokTile = 64;    // tokens per workgroup: 4 tiles of 16 of the prepared x
+constexpr uint32_t kBand = 4;        // token tiles of a band of the tile order
 constexpr uint32_t kSxtLorBlocks = 8;    // Q6_K: blocks of k up to which lo times r is taken too
 
 template <int TYPE>
@@ -367,13 +367,19 @@ __global__ __launch_bounds__(512) void k_sxt(WeightView wv, const uint8_t *__res
   const uint32_t tid = threadIdx.x, lane = tid & 63u, j = lane & 31u, h = lane >> 5;
   const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6), rg = wave & 3u, ks = wave >> 2;
 
-  // Workgroups of one XCD (blockIdx % 8) take a contiguous run of (k slice,
-  // tile) pairs, token tiles fastest: they share weights through its L2.
+  // Workgroups of one XCD (blockIdx % 8) take a contiguous run of (k slice, tile)
+  // pairs, in bands of 4 token tiles, token tiles fastest: the 32 tiles an XCD has
+  // at a time are 4 x 8, and share x and weights through its L2. Over all token
+  // tiles at once every CU read x of its own (us, Q4_K 8192 x 2048 at 2048 tokens 219
+  // / bands of 4 193 / of 8 194, IQ2_XXS 210 / 193 / 192, Q4_K 4096 x 4096 at 1500 145 /
+  // 141 / 139, 8192 x 2048 at 700 74.3 / 74.4 / 75.4, at 512 53.7 all).
   const uint32_t ntiles = row_tiles * tok_tiles, nwg = ntiles * ksl;
   uint32_t u = blockIdx.x;
   if (nwg % 8u == 0u) u = (blockIdx.x % 8u) * (nwg / 8u) + blockIdx.x / 8u;
   const uint32_t z = u / ntiles, lin = u - z * ntiles;
-  const uint32_t tt0 = lin % tok_tiles, r0 = (lin / tok_tiles) * 128u + 32u * rg;
+  const uint32_t band = lin / (kBand * row_tiles), bi = lin - band * kBand * row_tiles;
+  const uint32_t bw = min(kBand, tok_tiles - kBand * band);   // the last band's may be fewer
+  const uint32_t tt0 = kBand * band + bi % bw, r0 = (bi / bw) * 128u + 32u * rg;
   const uint32_t rows = wv.rows, nb = wv.k / 256u;
   const uint32_t bl = z * nb / ksl, bh = (z + 1u) * nb / ksl, iters = (bh - bl + 1u) / 2u;
 
