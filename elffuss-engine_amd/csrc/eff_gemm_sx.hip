@@ -865,7 +865,7 @@ uint32_t sx_tile_count(int type, uint32_t tokens) {
 // above the faster of the two summed, at most 6% above k_sx (Q6_K 4096 x 2048 at 80
 // tokens), and 16% (Q4_K), 40% (Q6_K), 12% (Q2_K) and 12% (IQ2_XXS) below k_sx alone.
 // us, k_sx / k_sxt: Q4_K 8192 x 2048 at 512 tokens 72.1 / 56.4, at 300 49.8 / 48.7, at
-// 2048 261 / 193, 4096 x 4096 at 1500 185 / 141; Q6_K 8192 x 2048 at 512 130 / 71, but
+// 2048 261 / 193, 4096 x 4096 at 1500 185 / 141; Q6_K 8192 x 2048 at 512 130 / 62, but
 // 2048 x 4096 at 80 20.0 / 23.4 (8 slices).
 uint32_t sxt_choose(const WeightView &wv, uint32_t tokens, double rounds, uint32_t walk, bool sliced) {
   struct Fit {

@@ -39,12 +39,13 @@
 //
 // Q6_K: u = sc (q - 32) has up to 13 bits, so its fp16 rounding v = fp16(u) is
 // off by r = u - v in {-1, 0, 1}, and only where |u| > 2048. The product takes
-// hi and lo times v, hi times r, and, up to 8 blocks of k, lo times r (below 2^-22
-// of the term). Left out there it shows (1.00-1.08 of k_sx's error at k = 512 to
-// 2048, 0.96-1.01 with it); from 9 blocks the shorter chains of sums outweigh it
-// (0.87-0.91 at 3328, 0.71-0.73 at 8192). It costs a fourth matrix instruction
-// (8192 x 2048 at 512 tokens 62.9 / 69.7 us, k_sx 130). One fold per block instead of
-// 16, whose 24 vector instructions per matrix instruction bound k_sx there.
+// hi and lo times v, hi times r, and, below 8 blocks of k, lo times r (below 2^-22
+// of the term). Left out there it shows (weights of both signs: 1.04 of k_sx's error
+// at k = 512 and 1.03 at 1024, with it 1.00 and 0.99, 0.98 at 1792); from 8 blocks
+// the shorter chains of sums make up for it (1.00 at 2048, of one sign up to 1.03;
+// 0.88-0.91 at 2304, 0.71-0.73 at 8192). It costs a fourth matrix instruction (8192 x
+// 2048 at 512 tokens 62.9 / 69.7 us, k_sx 130). One fold per block instead of 16, whose
+// 24 vector instructions per matrix instruction bound k_sx there.
 //
 // What bounds it: no unit (Q4_K 8192 x 2048 at 512 tokens: matrix cores busy 37% of
 // the kernel's clocks at 1.9 GHz, vector instructions 40%, LDS 27%, L2 10 TB/s). A CU
@@ -328,7 +329,7 @@ __device__ __forceinline__ void wait_vm_lds() {
 
 constexpr uint32_t kTokTile = 64;    // tokens per workgroup: 4 tiles of 16 of the prepared x
 constexpr uint32_t kBand = 4;        // token tiles of a band of the tile order
-constexpr uint32_t kSxtLorBlocks = 8;    // Q6_K: blocks of k up to which lo times r is taken too
+constexpr uint32_t kSxtLorBlocks = 7;    // Q6_K: blocks of k up to which lo times r is taken too
 
 template <int TYPE>
 struct SxtLds {

@@ -17,7 +17,7 @@ REL = 2.0 ** -20
 
 # (type, rows, k, tokens): shapes at which the planner takes the shared tiles (held
 # to that by test_shapes_take_the_shared_tiles), whole and in 2 to 8 k slices; Q6_K
-# also up to 8 blocks of k, where it takes one product more
+# also below 8 blocks of k, where it takes one product more
 SHAPES = [("Q4_K", 641, 256, 2000), ("Q4_K", 1000, 4352, 1000), ("Q4_K", 513, 8192, 501), ("Q4_K", 777, 768, 4000),
           ("Q4_K", 3000, 2304, 449), ("Q4_K", 700, 4352, 1500), ("Q2_K", 641, 256, 2000),
           ("Q2_K", 513, 8192, 501), ("Q2_K", 777, 768, 4000),
