@@ -48,7 +48,7 @@
 // 24 vector instructions per matrix instruction bound k_sx there.
 //
 // What bounds it: no unit (Q4_K 8192 x 2048 at 512 tokens: matrix cores busy 37% of
-// the kernel's clocks at 1.9 GHz, vector instructions 40%, LDS 27%, L2 10 TB/s). A CU
+// the kernel's clocks at 1.9 GHz, vector instructions 41%, LDS 27%, L2 10 TB/s). A CU
 // holds one workgroup, and nothing covers its first loads (about 4 us), the barrier
 // per group, the chain at a block's start and its end. us, k_sx and this kernel, both
 // with the preparation of x: Q4_K 8192 x 2048 at 512 tokens 72.1 / 56.4, at 1000 150.0 /
